@@ -170,6 +170,11 @@ struct WaveRanges {
     }
 };
 
+// Whether every numerator of WaveRanges fits 32 bits (as it does at any practical size).
+__device__ __forceinline__ bool ranges_narrow(int64_t total, int64_t n, int w) {
+    return (uint64_t)total * (uint64_t)(32 * n + w + 32) <= 0xffffffffull;
+}
+
 // One wave per workgroup; each wave owns one contiguous range of the chunk list. D is the head
 // dim, 128 or 64. A lane's K/V share of a 16-token tile is rows 4lg .. 4lg + 3 at 16-byte
 // (D 128: dims 8lc ..) or 8-byte (D 64: dims 4lc ..) width, so a wave reads whole rows.
@@ -188,8 +193,28 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
     __shared__ __attribute__((aligned(16))) unsigned char kt[16 * KP];  // one K tile
     const int lane = threadIdx.x, lg = lane >> 4, lc = lane & 15;
 
-    // ---- exclusive prefix sum of per-sequence chunk counts (each lane scans a slice)
-    {
+    // ---- exclusive prefix sum of per-sequence chunk counts. Up to 64 sequences stay in
+    // registers, one per lane (clamped context length and prefix), so that locating a segment
+    // is a ballot and scalar lane reads: no LDS search, no second read of a context length.
+    // (16-token pages: with other page sizes those two registers spill)
+    const bool in_lanes = BS16 && batch <= 64;
+    int my_ctx = 0, my_pre = 0, all_chunks;
+    if (in_lanes) {
+        my_ctx = lane < batch ? min(context_lens[lane], max_ctx) : 0;
+        const int n = decode_chunks(my_ctx, max_ctx);
+        const int incl = wave_incl_sum(n);
+        my_pre = incl - n;
+        all_chunks = __builtin_amdgcn_readlane(incl, 63);
+        if constexpr (FUSE) {  // its walk over the pairs reads them by index
+            if (lane < batch) pre[lane] = my_pre;
+            if (lane == 63) pre[batch] = incl;
+            __syncthreads();
+        }
+        if (blockIdx.x == 0) {  // for the merge kernel (ordered by the kernel boundary)
+            if (lane < batch) ws.pre[lane] = my_pre;
+            if (lane == 63) ws.pre[batch] = incl;
+        }
+    } else {  // each lane scans a slice, through LDS
         const int per = (batch + 63) / 64;
         int local = 0;
         for (int i = 0; i < per; i++) {
@@ -207,15 +232,35 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
         }
         if (lane == 63) pre[batch] = incl;
         __syncthreads();
-        if (blockIdx.x == 0)  // for the merge kernel (ordered by the kernel boundary)
+        all_chunks = __builtin_amdgcn_readlane(incl, 63);
+        if (blockIdx.x == 0)
             for (int b = lane; b <= batch; b += 64) ws.pre[b] = pre[b];
     }
-    const int64_t total = (int64_t)kv_heads * pre[batch];
+    const int64_t total = (int64_t)kv_heads * all_chunks;
     const int64_t nwg = gridDim.x, wgi = blockIdx.x;
-    const WaveRanges<int64_t> wr(total, nwg, ws.xcd_w);
-    const int64_t lo = wr.lo(wgi), hi = wr.lo(wgi + 1);
+    // 32-bit divisions whenever they fit: a 64-bit one is ~0.3 us of instructions, and the
+    // range bounds and the first segments stand before the wave's first load
+    const bool narrow = ranges_narrow(total, nwg, ws.xcd_w);
+    // The range is [lo, lo + len); positions in it are 32-bit offsets from lo
+    // (a range of 2^31 chunks would be 16 TB of reads). Everything that selects a segment is
+    // uniform and made scalar here: a divergent value would put every
+    // buffer load that takes its offset into a per-lane loop.
+    int64_t lo;
+    int len;
+    if (narrow) {
+        const WaveRanges<uint32_t> wr(total, nwg, ws.xcd_w);
+        const uint32_t a = wr.lo((uint32_t)wgi);
+        lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)a);
+        len = __builtin_amdgcn_readfirstlane((int)(wr.lo((uint32_t)wgi + 1) - a));
+    } else {
+        const WaveRanges<int64_t> wr(total, nwg, ws.xcd_w);
+        const int64_t a = wr.lo(wgi);
+        lo = ((int64_t)__builtin_amdgcn_readfirstlane((int)(a >> 32)) << 32) |
+             (uint32_t)__builtin_amdgcn_readfirstlane((int)a);
+        len = __builtin_amdgcn_readfirstlane((int)(wr.lo(wgi + 1) - a));
+    }
 
-    if (lo >= hi) return;
+    if (len <= 0) return;
 
     const uint32_t head_bytes = (uint32_t)(num_slots * D * (int64_t)sizeof(T));
     // K and V: instruction j of a tile reads rows 4lg + j, dims (D / 16) lc .. (4 whole rows)
@@ -227,23 +272,36 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
     struct Seg {
         int b, g, cb, ce, nch, tok_end;
     };
-    auto seg_at = [&](int64_t x) -> Seg {
-        int l0 = 0, h0 = batch;  // largest b with kv_heads * pre[b] <= x
-        while (h0 - l0 > 1) {
-            const int mid = (l0 + h0) >> 1;
-            if ((int64_t)kv_heads * pre[mid] <= x)
-                l0 = mid;
-            else
-                h0 = mid;
-        }
+    auto seg_at = [&](int at) -> Seg {
+        const int64_t x = lo + at;
         Seg sg;
-        sg.b = l0;
-        sg.nch = pre[l0 + 1] - pre[l0];
-        const int64_t rel = x - (int64_t)kv_heads * pre[l0];
-        sg.g = (int)(rel / sg.nch);
+        int before, ctx;  // chunks per head before sequence b, its clamped context length
+        if (in_lanes) {   // largest b with kv_heads * pre[b] <= x
+            const uint64_t le = __ballot(lane < batch && (int64_t)kv_heads * my_pre <= x);
+            sg.b = __popcll(le) - 1;
+            before = __builtin_amdgcn_readlane(my_pre, sg.b);
+            ctx = __builtin_amdgcn_readlane(my_ctx, sg.b);
+            sg.nch = decode_chunks(ctx, max_ctx);
+        } else {
+            int l0 = 0, h0 = batch;
+            while (h0 - l0 > 1) {
+                const int mid = (l0 + h0) >> 1;
+                if ((int64_t)kv_heads * pre[mid] <= x)
+                    l0 = mid;
+                else
+                    h0 = mid;
+            }
+            sg.b = __builtin_amdgcn_readfirstlane(l0);
+            before = __builtin_amdgcn_readfirstlane(pre[l0]);
+            sg.nch = __builtin_amdgcn_readfirstlane(pre[l0 + 1]) - before;
+            ctx = min(context_lens[sg.b], max_ctx);
+        }
+        const int64_t rel = x - (int64_t)kv_heads * before;
+        sg.g = __builtin_amdgcn_readfirstlane(narrow ? (int)((uint32_t)rel / (uint32_t)sg.nch)
+                                                     : (int)(rel / sg.nch));
         sg.cb = (int)(rel - (int64_t)sg.g * sg.nch);
-        sg.ce = (int)min(min((int64_t)sg.nch, (int64_t)sg.cb + DEC_SEG), sg.cb + (hi - x));
-        sg.tok_end = min(min(context_lens[sg.b], max_ctx), sg.ce * DEC_CHUNK);
+        sg.ce = sg.cb + min(min(sg.nch - sg.cb, DEC_SEG), len - at);
+        sg.tok_end = min(ctx, sg.ce * DEC_CHUNK);
         return sg;
     };
     // Pool slot of the first token of each tile of a segment: lane i holds tile i (chunk
@@ -262,7 +320,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
         const int last_tile_tok0 = ((sg.tok_end - 1) >> 4) << 4;
         const int tok0 = min(sg.cb * DEC_CHUNK + lane * 16, last_tile_tok0);
         const int lb = BS16 ? (tok0 >> 4) : tok0 / block_size;
-        return Slots{bt[lb], tok0 - lb * block_size};
+        return Slots{bt[lb], BS16 ? 0 : tok0 - lb * block_size};
     };
     // Chunk loads as buffer loads: one resource per pool (the kv head's region), the
     // loop-invariant lane offset (VGPR) and the tile's byte offset (SGPR), so there is no
@@ -277,9 +335,10 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
         for (int t = 0; t < 2; t++) {
             int id = __builtin_amdgcn_readlane(sl.id, tile0 + t);
             id = id < 0 ? 0 : (id > max_id ? max_id : id);  // a bad block id never leaves the pool
-            const uint32_t soff =
-                (uint32_t)(id * block_size + __builtin_amdgcn_readlane(sl.off, tile0 + t)) *
-                (uint32_t)(D * sizeof(T));
+            const uint32_t slot =
+                BS16 ? (uint32_t)(id * 16)
+                     : (uint32_t)(id * block_size + __builtin_amdgcn_readlane(sl.off, tile0 + t));
+            const uint32_t soff = slot * (uint32_t)(D * sizeof(T));
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 if constexpr (D == 128)
@@ -408,11 +467,11 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
     // (r < 4, nn < NV): D / 4 contiguous dims.
     auto epilogue = [&](int b, int g, bool complete, bool first_piece) {
         lsum = sum_across_rows(lsum);
-        // FUSE: lg made opaque here, so the per-lane output addresses are formed at the store
-        // instead of being hoisted out of the stream as 64-bit values (which spill in that
-        // instantiation, and a spill reload waits for every chunk load in flight)
+        // lg made opaque here, so the per-lane output addresses are formed at the store instead
+        // of being hoisted out of the stream as 64-bit values (which spill, and a spill reload
+        // waits for every chunk load in flight)
         int lgo = lg;
-        if constexpr (FUSE) asm volatile("" : "+v"(lgo));
+        asm volatile("" : "+v"(lgo));
         if (lc < n_rep) {
             if (complete) {  // whole pair in this range: final output
                 const int64_t row = ws.rows ? (int64_t)ws.rows[b] : (int64_t)b;
@@ -476,8 +535,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
     struct NewRows {
         int b, g, slot[2], pb[2], pg[2];
         bool pv[2], more;
-        int64_t first;
-        int nch;
+        int first, nch;
         Ld kr[2], vr[2];
     };
     auto new_rows_load = [&](NewRows& nr) {
@@ -496,7 +554,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
                 }
                 if (nr.b < batch) {
                     nr.nch = pre[nr.b + 1] - pre[nr.b];
-                    nr.more = nr.first + nr.nch - 1 < hi;
+                    nr.more = nr.first + nr.nch - 1 < len;
                 } else {
                     nr.more = false;
                 }
@@ -529,19 +587,19 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
         }
     };
 
-    Seg cur = seg_at(lo);
+    Seg cur = seg_at(0);
     NewRows nr{};
     if constexpr (FUSE) {
         nr.b = cur.b;
         nr.g = cur.g;
         nr.nch = cur.nch;
-        nr.first = lo - cur.cb;  // flattened position of pair (b, g)'s first chunk
-        nr.more = nr.first + nr.nch - 1 < hi;
+        nr.first = -cur.cb;  // pair (b, g)'s first chunk, as an offset from lo
+        nr.more = nr.first + nr.nch - 1 < len;
         new_rows_load(nr);
     }
     Slots cur_slots = seg_slots(cur);
-    int64_t nx = lo + (cur.ce - cur.cb);
-    bool has_nxt = nx < hi;
+    int nx = cur.ce - cur.cb;
+    bool has_nxt = nx < len;
     Seg nxt = cur;
     Slots nxt_slots = cur_slots;
     if (has_nxt) {
@@ -561,13 +619,13 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
         // At a segment's last chunk the segment after the next one is looked up and its
         // block-table entries are requested before this step's chunk loads, so the rotation at
         // the end of the step waits for that load alone and not for the chunk loads behind it.
-        int64_t nn_x = nx;
+        int nn_x = nx;
         bool has_nn = false;
         Seg nn = nxt;
         Slots nn_slots = nxt_slots;
         if (seg_end && has_nxt) {
             nn_x = nx + (nxt.ce - nxt.cb);
-            has_nn = nn_x < hi;
+            has_nn = nn_x < len;
             if (has_nn) {
                 nn = seg_at(nn_x);
                 nn_slots = seg_slots(nn);
@@ -619,7 +677,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
     using pf_off = std::integral_constant<bool, false>;
     Ld ka[2][4], va[2][4], kb[2][4], vb[2][4];
     load_chunk(cur.g, cur_slots, 0, ka, va);
-    int64_t remaining = hi - lo;  // chunks this wave computes; all but the last prefetch one
+    int remaining = len;  // chunks this wave computes; all but the last prefetch one
     for (; remaining > 2; remaining -= 2) {
         step(pf_on{}, ka, va, kb, vb);
         step(pf_on{}, kb, vb, ka, va);
@@ -632,36 +690,39 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
     }
 }
 
-// Merge of the pieces of pairs cut by wave ranges, and zero rows for empty contexts: one wave
-// per (query head, sequence), lane i owning output dims 2i and 2i + 1, locating its pieces from
-// the chunk prefix sums the main kernel left in the workspace. Pieces are taken 64 at a time
-// (one per lane): their (max, sum) pairs become weights through wave reductions, then every
+// Merge of the pieces of pairs cut by wave ranges, and zero rows for empty contexts: one
+// workgroup per (query head, sequence), lane i owning output dims 2i and 2i + 1, locating its
+// pieces from the chunk prefix sums the main kernel left in the workspace. Pieces are taken 64 at
+// a time (one per lane): their (max, sum) pairs become weights through wave reductions, then every
 // lane accumulates its two dims over the batch with independent loads, reading each piece's
 // weight and slot from the lane that holds it; batches combine with the same online rescaling
-// as the running update of cpu.rs:96-105. No LDS and no barrier.
+// as the running update of cpu.rs:96-105. With many pieces per pair (few sequences) the
+// workgroup's waves split them, since one wave reads them 8 rows a memory round trip, and fold
+// their states through LDS; with one wave there is no LDS and no barrier.
+static constexpr int DEC_MERGE_WAVES = 8;
 template <typename TO, int D>
-__global__ __launch_bounds__(64) void paged_decode_merge_kernel(
+__global__ __launch_bounds__(64 * DEC_MERGE_WAVES) void paged_decode_merge_kernel(
     TO* __restrict__ out, int batch, int num_heads, int kv_heads, int n_rep, int nwg_i,
     DecodeWs ws) {
     // lane i owns output dims E i .. E i + E - 1
     constexpr int E = D / 64;
-    const int h = blockIdx.x, b = blockIdx.y, lane = threadIdx.x;
+    const int h = blockIdx.x, b = blockIdx.y, lane = threadIdx.x & 63;
+    const int w_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     // chunks before sequence b, of sequence b and in all sequences (the main kernel's sums)
     const int before = ws.pre[b], nch = ws.pre[b + 1] - before, all = ws.pre[batch];
     const int64_t orow = ws.rows ? (int64_t)ws.rows[b] : (int64_t)b;
     TO* o = out + (orow * num_heads + h) * D + E * lane;
     if (nch == 0) {
+        if (w_id == 0)
 #pragma unroll
-        for (int i = 0; i < E; i++) o[i] = from_f32<TO>(0.0f);
+            for (int i = 0; i < E; i++) o[i] = from_f32<TO>(0.0f);
         return;
     }
     const int g = h / n_rep, hh = h - g * n_rep;
     const int64_t total = (int64_t)kv_heads * all, nwg = nwg_i;
     const int64_t s = (int64_t)kv_heads * before + (int64_t)g * nch;
     const int64_t e = s + nch;
-    // Range owners and bounds, in 32-bit arithmetic whenever chunks x (W + 32) fits (it bounds
-    // every numerator of WaveRanges), as it does at any practical size.
-    const bool narrow = (uint64_t)total * (uint64_t)(32 * nwg + ws.xcd_w + 32) <= 0xffffffffull;
+    const bool narrow = ranges_narrow(total, nwg, ws.xcd_w);
     const WaveRanges<uint32_t> r32(narrow ? total : 1, nwg, ws.xcd_w);
     const WaveRanges<int64_t> r64(total, nwg, ws.xcd_w);
     auto range_lo = [&](int64_t i) -> int64_t {
@@ -697,17 +758,20 @@ __global__ __launch_bounds__(64) void paged_decode_merge_kernel(
             O[0] += wj * v;
         }
     };
-    for (int p0 = 0; p0 < np; p0 += 64) {
+    // this wave's pieces: an equal share
+    const int per = waves == 1 ? np : (np + waves - 1) / waves;
+    const int p_end = min(np, (w_id + 1) * per);
+    for (int p0 = w_id * per; p0 < p_end; p0 += 64) {
         // The batch's first 8 pieces' rows are loaded before the (max, sum) reductions, which
         // they do not depend on (a missing piece reads the first piece's row, weight 0).
         RowV v0[8];
         int s0[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            s0[j] = p0 + j < np ? piece_slot(p0 + j) : -1;
+            s0[j] = p0 + j < p_end ? piece_slot(p0 + j) : -1;
             v0[j] = row(s0[j] >= 0 ? s0[j] : fslot);
         }
-        const int slot = p0 + lane < np ? piece_slot(p0 + lane) : -1;
+        const int slot = p0 + lane < p_end ? piece_slot(p0 + lane) : -1;
         float mx = -INFINITY, lx = 0.0f;
         if (slot >= 0) {
             mx = ws.ml[2 * ((int64_t)slot * n_rep + hh)];
@@ -728,7 +792,7 @@ __global__ __launch_bounds__(64) void paged_decode_merge_kernel(
         // The rest in groups of 8 unconditional loads (a missing piece reads the first piece's
         // row) so they are all in flight together; the select drops them, so stale workspace
         // bits (even NaN) never reach the sum.
-        const int nb = min(64, np - p0);
+        const int nb = min(64, p_end - p0);
         for (int q = 8; q < nb; q += 8) {
             RowV v[8];
             int sl[8];
@@ -745,8 +809,42 @@ __global__ __launch_bounds__(64) void paged_decode_merge_kernel(
         }
         M = m_new;
     }
+    if (waves > 1) {  // the waves' states, folded by the first (a wave without pieces has M = -inf)
+        __shared__ float wM[DEC_MERGE_WAVES], wL[DEC_MERGE_WAVES];
+        __shared__ float wO[DEC_MERGE_WAVES][E][64];
+        if (lane == 0) {
+            wM[w_id] = M;
+            wL[w_id] = L;
+        }
+#pragma unroll
+        for (int i = 0; i < E; i++) wO[w_id][i][lane] = O[i];
+        __syncthreads();
+        if (w_id != 0) return;
+        float Mt = M;
+        for (int x = 1; x < waves; x++) Mt = fmaxf(Mt, wM[x]);
+        const float f0 = fast_exp2(M - Mt);
+        L *= f0;
+#pragma unroll
+        for (int i = 0; i < E; i++) O[i] *= f0;
+        for (int x = 1; x < waves; x++) {
+            if (x * per >= np) break;  // no pieces there
+            const float f = fast_exp2(wM[x] - Mt);
+            L += wL[x] * f;
+#pragma unroll
+            for (int i = 0; i < E; i++) O[i] += wO[x][i][lane] * f;
+        }
+    }
 #pragma unroll
     for (int i = 0; i < E; i++) o[i] = from_f32<TO>(O[i] / L);
+}
+
+// Waves per merge workgroup: about eight pieces (one memory round trip) each, for the mean number
+// of pieces per pair and twice that on the longest contexts.
+static int decode_merge_waves(int nwg, int batch, int kv_heads) {
+    const int64_t pieces = 2 * (int64_t)nwg / ((int64_t)batch * kv_heads);
+    int waves = 1;
+    while (waves < DEC_MERGE_WAVES && 8 * waves < pieces) waves *= 2;
+    return waves;
 }
 
 template <typename T, typename TO, int D>
@@ -770,7 +868,8 @@ static int launch_decode_mfma_d(void* out, const void* q, const void* k_pool, co
         block_size, num_slots, max_ctx, scale * LOG2E, ws);
     int rc = check_hip(hipGetLastError(), "paged_decode launch");
     if (rc != FLOUR_OK) return rc;
-    paged_decode_merge_kernel<TO, D><<<dim3(num_heads, batch), dim3(64), 0, stream>>>(
+    const int mw = decode_merge_waves(nwg, batch, kv_heads);
+    paged_decode_merge_kernel<TO, D><<<dim3(num_heads, batch), dim3(64 * mw), 0, stream>>>(
         static_cast<TO*>(out), batch, num_heads, kv_heads, n_rep, nwg, ws);
     return check_hip(hipGetLastError(), "paged_decode merge launch");
 }
