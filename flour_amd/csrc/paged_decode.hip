@@ -38,6 +38,11 @@
 //    O^T accumulator holds, in lane (g, c), query head c at dims 32g..32g+31.
 //  * P is split into hi + lo 16-bit parts (two MFMAs per product) so the P.V contraction keeps
 //    ~16 mantissa bits of P; products are exact in fp32 and accumulate in fp32.
+//  * fp32 pools (longer steps, decode_f32_split): the same stream over 16-token chunks of the same
+//    bytes, on v_mfma_f32_16x16x4 in fp32 end to end. A wave instruction reads four 256 B row
+//    segments; the score registers are the B operand as they stand (one product per token group
+//    and 16 dims) and V registers the A operand, so only K goes through LDS. HBM-bound: 16 x
+//    256-2,048 tokens of 32 / 8 heads of 128 (129 MB) 108 us on the vector kernel, 36.8 here.
 //  * Online softmax in the exp2 domain: the only cross-lane step per chunk is the max over the
 //    four row groups (two v_permlane*_swap exchanges); running sums stay lane-partial until
 //    the end, and the accumulator is rescaled only when some lane's max moved.
@@ -68,8 +73,9 @@ int launch_attn_generic(int dtype, int out_dtype, void* out, int64_t o_st, int64
 
 static constexpr float LOG2E = 1.4426950408889634f;
 
-static constexpr int DEC_CHUNK = 32;         // tokens per step (two 16-token MFMA tiles)
-static constexpr int DEC_SEG = 32;           // chunks per tile-slot refill (64 tiles, one per lane)
+// Tokens per step: two 16-token MFMA tiles of a 16-bit pool, one of an fp32 pool (the same bytes)
+__host__ __device__ constexpr int dec_chunk(int elem_bytes) { return elem_bytes == 4 ? 16 : 32; }
+static constexpr int DEC_SEG = 32;           // chunks per tile-slot refill (up to 64 tiles, one per lane)
 static constexpr int DEC_MAX_BATCH = 4096;   // per-sequence chunk prefix sums live in LDS
 // Three waves per CU. Each wave keeps one 32-token chunk in flight while it computes the
 // previous one (16 KB at head_dim 128), so 768 waves hold ~12 MB of reads, about HBM's
@@ -78,13 +84,18 @@ static constexpr int DEC_MAX_BATCH = 4096;   // per-sequence chunk prefix sums l
 // 3 per CU stream 0.3-1.5% faster than 4, which stream 3-7% faster than 8; counts that do not
 // divide evenly over a CU's 4 SIMDs, 2.5, 3.5 and 5 per CU, are slower than their neighbours).
 static constexpr int DEC_WAVES_PER_CU = 3;
+// fp32 pools: the fp32 products of a chunk keep a SIMD's matrix core busy for ~2,050 cycles of
+// every 16 KB, so every SIMD gets a wave (3 / 4 / 6 per CU: 163 / 149 / 142 us for 855 MB at 32 / 8
+// heads of 128, 131 / 126 / 136 us for 806 MB at 8 heads of 64).
+static constexpr int DEC_WAVES_PER_CU_F32 = 4;
+static_assert(DEC_WAVES_PER_CU_F32 >= DEC_WAVES_PER_CU, "the workspace is sized for the larger");
 // K is read like V, four whole 256 B rows per instruction with the non-temporal hint, and
 // turned into the MFMA A-operand layout (row = lane % 16) through a per-wave LDS tile. Reading
 // K directly in that layout takes a 64 B quarter of 16 rows per instruction, a pattern that
 // streams at most ~6.0 TB/s from HBM against ~6.8 TB/s for whole rows (measured with the same
 // 2048-wave, double-buffered access over random 4 KB runs).
-// Bytes per K row in LDS (head_dim 128 / 64): conflict-free 16-byte fragment reads of 16 rows.
-__host__ __device__ constexpr int dec_kpitch(int d) { return d == 128 ? 272 : 144; }
+// Bytes per K row in LDS: the row and 16 bytes, conflict-free 16-byte fragment reads of 16 rows.
+__host__ __device__ constexpr int dec_kpitch(int d, int elem_bytes) { return d * elem_bytes + 16; }
 
 struct DecodeWs {
     float* ml;  // [2 * num_waves][n_rep][2] (max, sum) in the exp2 domain
@@ -126,8 +137,9 @@ static int device_cus() {
     return cached[dev];
 }
 
-static int decode_workgroups() {
-    const int n = g_wg_override > 0 ? g_wg_override : device_cus() * DEC_WAVES_PER_CU;
+static int decode_workgroups(int dtype) {
+    const int per_cu = dtype == FLOUR_DTYPE_F32 ? DEC_WAVES_PER_CU_F32 : DEC_WAVES_PER_CU;
+    const int n = g_wg_override > 0 ? g_wg_override : device_cus() * per_cu;
     return n < 4096 ? n : 4096;
 }
 
@@ -140,9 +152,10 @@ static size_t decode_ws_bytes(int nwg, int n_rep, int head_dim, int batch) {
            align256(((size_t)batch + 1) * sizeof(int));
 }
 
+template <int CHUNK>
 __device__ __forceinline__ int decode_chunks(int ctx, int max_ctx) {
     ctx = min(ctx, max_ctx);
-    return ctx > 0 ? (ctx + DEC_CHUNK - 1) / DEC_CHUNK : 0;
+    return ctx > 0 ? (ctx + CHUNK - 1) / CHUNK : 0;
 }
 
 // Wave ranges over the flattened chunk list. The dispatcher places workgroup i on XCD i % 8,
@@ -175,6 +188,19 @@ __device__ __forceinline__ bool ranges_narrow(int64_t total, int64_t n, int w) {
     return (uint64_t)total * (uint64_t)(32 * n + w + 32) <= 0xffffffffull;
 }
 
+// Ranges that a list of `total` chunks is cut into by a grid of `cap` waves: at least two chunks
+// each. Fewer, longer ranges leave fewer pieces to merge (one 2,000-token sequence of 8 kv heads,
+// 504 chunks: 10.2 us on 256 waves, 10.9 on 504), a list of more than `cap` chunks has a range of
+// two anyway, and no range is empty (the smallest share is (32 - w) / 32 >= 1/2 of the mean).
+__device__ __forceinline__ int64_t range_count(int64_t total, int64_t cap) {
+    const int64_t half = total >> 1;
+    return half < 1 ? 1 : (half < cap ? half : cap);
+}
+
+__device__ __forceinline__ f32x4 mfma16x16x4_f32(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
 // One wave per workgroup; each wave owns one contiguous range of the chunk list. D is the head
 // dim, 128 or 64. A lane's K/V share of a 16-token tile is rows 4lg .. 4lg + 3 at 16-byte
 // (D 128: dims 8lc ..) or 8-byte (D 64: dims 4lc ..) width, so a wave reads whole rows.
@@ -185,10 +211,16 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
     const int32_t* __restrict__ context_lens, int batch, int num_heads, int kv_heads, int n_rep,
     int block_size, int64_t num_slots, int max_ctx, float scale_log2, DecodeWs ws) {
     static_assert(D == 128 || D == 64, "matrix-core decode: head_dim 128 or 64");
-    constexpr int KP = dec_kpitch(D);
+    constexpr bool F32 = std::is_same<T, float>::value;
+    constexpr int CHUNK = dec_chunk(sizeof(T));
+    constexpr int TILES = CHUNK / 16;  // 16-token tiles per chunk
+    constexpr int KP = dec_kpitch(D, sizeof(T));
     constexpr int NV = D / 16;  // O^T products per chunk (16 output dims each)
-    // a lane's load of one row: 8 (D 128) or 4 (D 64) dims
-    typedef typename std::conditional<D == 128, u32x4, u32x2>::type Ld;
+    // A lane's loads of K (and of V) per chunk: [NL][4] of Ld. 16-bit pools: tile t, row 4lg + j,
+    // 8 (D 128) or 4 (D 64) dims. fp32 pools: row 4lg + j of the one tile, dims 64i + 4lc .. + 3,
+    // so an instruction reads four 256-byte row segments in every form (128 at D 64, 16-bit).
+    constexpr int NL = F32 ? D / 64 : TILES;
+    typedef typename std::conditional<F32 || D == 128, u32x4, u32x2>::type Ld;
     extern __shared__ int pre[];  // pre[b] = chunks of sequences 0..b-1; pre[batch] = all
     __shared__ __attribute__((aligned(16))) unsigned char kt[16 * KP];  // one K tile
     const int lane = threadIdx.x, lg = lane >> 4, lc = lane & 15;
@@ -201,7 +233,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
     int my_ctx = 0, my_pre = 0, all_chunks;
     if (in_lanes) {
         my_ctx = lane < batch ? min(context_lens[lane], max_ctx) : 0;
-        const int n = decode_chunks(my_ctx, max_ctx);
+        const int n = decode_chunks<CHUNK>(my_ctx, max_ctx);
         const int incl = wave_incl_sum(n);
         my_pre = incl - n;
         all_chunks = __builtin_amdgcn_readlane(incl, 63);
@@ -219,7 +251,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
         int local = 0;
         for (int i = 0; i < per; i++) {
             const int b = lane * per + i;
-            if (b < batch) local += decode_chunks(context_lens[b], max_ctx);
+            if (b < batch) local += decode_chunks<CHUNK>(context_lens[b], max_ctx);
         }
         const int incl = wave_incl_sum(local);
         int run = incl - local;
@@ -227,7 +259,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
             const int b = lane * per + i;
             if (b < batch) {
                 pre[b] = run;
-                run += decode_chunks(context_lens[b], max_ctx);
+                run += decode_chunks<CHUNK>(context_lens[b], max_ctx);
             }
         }
         if (lane == 63) pre[batch] = incl;
@@ -237,7 +269,8 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
             for (int b = lane; b <= batch; b += 64) ws.pre[b] = pre[b];
     }
     const int64_t total = (int64_t)kv_heads * all_chunks;
-    const int64_t nwg = gridDim.x, wgi = blockIdx.x;
+    const int64_t nwg = range_count(total, gridDim.x), wgi = blockIdx.x;
+    if (total == 0 || wgi >= nwg) return;
     // 32-bit divisions whenever they fit: a 64-bit one is ~0.3 us of instructions, and the
     // range bounds and the first segments stand before the wave's first load
     const bool narrow = ranges_narrow(total, nwg, ws.xcd_w);
@@ -260,11 +293,12 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
         len = __builtin_amdgcn_readfirstlane((int)(wr.lo(wgi + 1) - a));
     }
 
-    if (len <= 0) return;
-
     const uint32_t head_bytes = (uint32_t)(num_slots * D * (int64_t)sizeof(T));
     // K and V: instruction j of a tile reads rows 4lg + j, dims (D / 16) lc .. (4 whole rows)
-    const uint32_t v_off = (uint32_t)((4 * lg * D + (D / 16) * lc) * sizeof(T));
+    uint32_t v_off = (uint32_t)((4 * lg * D + (F32 ? 4 : D / 16) * lc) * sizeof(T));
+    // opaque: with its low bits known, the row offsets become ORs held in a register each instead
+    // of the loads' immediate offsets
+    asm volatile("" : "+v"(v_off));
     const int64_t max_phys = num_slots / block_size - 1;
 
     // The wave's range is a stream of segments: up to DEC_SEG consecutive chunks of one
@@ -281,7 +315,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
             sg.b = __popcll(le) - 1;
             before = __builtin_amdgcn_readlane(my_pre, sg.b);
             ctx = __builtin_amdgcn_readlane(my_ctx, sg.b);
-            sg.nch = decode_chunks(ctx, max_ctx);
+            sg.nch = decode_chunks<CHUNK>(ctx, max_ctx);
         } else {
             int l0 = 0, h0 = batch;
             while (h0 - l0 > 1) {
@@ -301,7 +335,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
                                                      : (int)(rel / sg.nch));
         sg.cb = (int)(rel - (int64_t)sg.g * sg.nch);
         sg.ce = sg.cb + min(min(sg.nch - sg.cb, DEC_SEG), len - at);
-        sg.tok_end = min(ctx, sg.ce * DEC_CHUNK);
+        sg.tok_end = min(ctx, sg.ce * CHUNK);
         return sg;
     };
     // Pool slot of the first token of each tile of a segment: lane i holds tile i (chunk
@@ -318,7 +352,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
     auto seg_slots = [&](const Seg& sg) -> Slots {
         const int32_t* bt = block_tables + (int64_t)sg.b * max_blocks;
         const int last_tile_tok0 = ((sg.tok_end - 1) >> 4) << 4;
-        const int tok0 = min(sg.cb * DEC_CHUNK + lane * 16, last_tile_tok0);
+        const int tok0 = min(sg.cb * CHUNK + lane * 16, last_tile_tok0);
         const int lb = BS16 ? (tok0 >> 4) : tok0 / block_size;
         return Slots{bt[lb], BS16 ? 0 : tok0 - lb * block_size};
     };
@@ -332,41 +366,42 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
         const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
             (void*)(v_pool + (int64_t)g * num_slots * D), (short)0, (int)head_bytes, BUF_DWORD3);
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
+        for (int t = 0; t < TILES; t++) {
             int id = __builtin_amdgcn_readlane(sl.id, tile0 + t);
             id = id < 0 ? 0 : (id > max_id ? max_id : id);  // a bad block id never leaves the pool
             const uint32_t slot =
                 BS16 ? (uint32_t)(id * 16)
                      : (uint32_t)(id * block_size + __builtin_amdgcn_readlane(sl.off, tile0 + t));
             const uint32_t soff = slot * (uint32_t)(D * sizeof(T));
+            auto load_rows = [&](const __amdgpu_buffer_rsrc_t& rsrc, Ld (*d)[4]) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if constexpr (D == 128)
-                    kd[t][j] = __builtin_amdgcn_raw_buffer_load_b128(
-                        k_rsrc, v_off + j * D * (uint32_t)sizeof(T), soff, BUF_NT);
-                else
-                    kd[t][j] = __builtin_amdgcn_raw_buffer_load_b64(
-                        k_rsrc, v_off + j * D * (uint32_t)sizeof(T), soff, BUF_NT);
-            }
+                for (int i = 0; i < NL / TILES; i++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if constexpr (D == 128)
-                    vd[t][j] = __builtin_amdgcn_raw_buffer_load_b128(
-                        v_rsrc, v_off + j * D * (uint32_t)sizeof(T), soff, BUF_NT);
-                else
-                    vd[t][j] = __builtin_amdgcn_raw_buffer_load_b64(
-                        v_rsrc, v_off + j * D * (uint32_t)sizeof(T), soff, BUF_NT);
-            }
+                    for (int j = 0; j < 4; j++) {
+                        const uint32_t off = v_off + (j * D + 64 * i) * (uint32_t)sizeof(T);
+                        if constexpr (sizeof(Ld) == 16)
+                            d[t + i][j] =
+                                __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, soff, BUF_NT);
+                        else
+                            d[t + i][j] =
+                                __builtin_amdgcn_raw_buffer_load_b64(rsrc, off, soff, BUF_NT);
+                    }
+            };
+            load_rows(k_rsrc, kd);
+            load_rows(v_rsrc, vd);
         }
     };
-    // Q^T as the B operand: lane (lg, lc) holds head lc, dims 32kk + 8lg .. +7.
-    u32x4 qb[D / 32];
+    // Q^T as the B operand: lane (lg, lc) holds head lc, dims 32kk + 8lg .. +7; fp32: dims
+    // 16kk + 4lg .. + 3, one per k-step 4kk .. 4kk + 3.
+    constexpr int NQ = D * (int)sizeof(T) / 64;
+    u32x4 qb[NQ];
     auto load_q = [&](int b, int g) {
         const int64_t row = ws.rows ? (int64_t)ws.rows[b] : (int64_t)b;
-        const T* qh = q + (row * num_heads + (int64_t)g * n_rep + lc) * D + 8 * lg;
+        const T* qh = q + (row * num_heads + (int64_t)g * n_rep + lc) * D + (F32 ? 4 : 8) * lg;
 #pragma unroll
-        for (int kk = 0; kk < D / 32; kk++)
-            qb[kk] = (lc < n_rep) ? *reinterpret_cast<const u32x4*>(qh + 32 * kk) : u32x4{0, 0, 0, 0};
+        for (int kk = 0; kk < NQ; kk++)
+            qb[kk] = (lc < n_rep) ? *reinterpret_cast<const u32x4*>(qh + (F32 ? 16 : 32) * kk)
+                                  : u32x4{0, 0, 0, 0};
     };
 
     float m = -INFINITY, lsum = 0.0f;
@@ -375,44 +410,69 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
     for (int nn = 0; nn < NV; nn++) acc[nn] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     auto compute_chunk = [&](int c, int tok_end, Ld (*ka)[4], Ld (*va)[4]) {
-        const int tok0 = c * DEC_CHUNK;
-        const bool full = tok0 + DEC_CHUNK <= tok_end;
+        const int tok0 = c * CHUNK;
+        const bool full = tok0 + CHUNK <= tok_end;
         if (!full) {  // tokens past the context: zero V so garbage bits cannot leak in
 #pragma unroll
-            for (int t = 0; t < 2; t++)
+            for (int t = 0; t < NL; t++)
 #pragma unroll
                 for (int j = 0; j < 4; j++)
-                    if (tok0 + 16 * t + 4 * lg + j >= tok_end) va[t][j] = Ld{};
+                    if (tok0 + (F32 ? 0 : 16 * t) + 4 * lg + j >= tok_end) va[t][j] = Ld{};
         }
         // K rows through LDS into the A-operand layout: lane (lg, lc) needs row lc, dims
-        // 32kk + 8lg .. +7. One wave per workgroup and LDS operations of a wave complete in
-        // order, so the wave barriers only keep the compiler from moving LDS accesses across.
-        // The second tile's writes follow the first tile's reads in that order.
-        u32x4 kA[2][D / 32];
+        // 32kk + 8lg .. +7 (fp32: 16kk + 4lg .. + 3). One wave per workgroup and LDS operations
+        // of a wave complete in order, so the wave barriers only keep the compiler from moving
+        // LDS accesses across. The second tile's writes follow the first tile's reads in that
+        // order.
+        u32x4 kA[TILES][NQ];
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
+        for (int t = 0; t < TILES; t++) {
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                *reinterpret_cast<Ld*>(&kt[(4 * lg + j) * KP + (int)sizeof(Ld) * lc]) = ka[t][j];
+            for (int i = 0; i < NL / TILES; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    *reinterpret_cast<Ld*>(&kt[(4 * lg + j) * KP + 256 * i + (int)sizeof(Ld) * lc]) =
+                        ka[t + i][j];
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int kk = 0; kk < D / 32; kk++)
+            for (int kk = 0; kk < NQ; kk++)
                 kA[t][kk] = *reinterpret_cast<const u32x4*>(&kt[lc * KP + 64 * kk + 16 * lg]);
         }
         __builtin_amdgcn_wave_barrier();
         // S tiles: s[t][r] = score of head lc for token 16t + 4lg + r of the chunk.
-        f32x4 s[2];
+        f32x4 s[TILES];
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
+        for (int t = 0; t < TILES; t++) {
             s[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (F32) {
+                // Sums of 8 products, added pairwise: one chain over the D products of a score has
+                // ~1.3 times the vector kernel's rounding error on short contexts.
+                f32x4 lvl[4];  // lvl[n]: a pending sum of 2^n k-steps
 #pragma unroll
-            for (int kk = 0; kk < D / 32; kk++) s[t] = mfma16x16x32<T>(kA[t][kk], qb[kk], s[t]);
+                for (int kk = 0; kk < NQ; kk++) {
+                    f32x4 h[2] = {s[t], s[t]};
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        h[e >> 1] = mfma16x16x4_f32(__uint_as_float(kA[t][kk][e]),
+                                                    __uint_as_float(qb[kk][e]), h[e >> 1]);
+                    f32x4 x = h[0] + h[1];
+                    int n = 0;
+                    for (; (kk >> n) & 1; n++) x = lvl[n] + x;
+                    lvl[n] = x;
+                    if (kk & 1) __builtin_amdgcn_sched_barrier(0);  // (few pending sums)
+                }
+                s[t] = lvl[NQ == 8 ? 3 : 2];
+                __builtin_amdgcn_sched_barrier(0);  // (registers: no V^T P^T before the scores)
+            } else {
+#pragma unroll
+                for (int kk = 0; kk < NQ; kk++) s[t] = mfma16x16x32<T>(kA[t][kk], qb[kk], s[t]);
+            }
         }
-        float sv[8];
+        float sv[4 * TILES];
         float tmax = -INFINITY;
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+        for (int t = 0; t < TILES; t++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const bool ok = full || (tok0 + 16 * t + 4 * lg + r < tok_end);
@@ -422,49 +482,68 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
         tmax = max_across_rows(tmax);
         const float m_new = fmaxf(m, tmax);
         const float alpha = fast_exp2(m - m_new);
-        float p[8];
+        float p[4 * TILES];
 #pragma unroll
-        for (int i = 0; i < 8; i++) p[i] = fast_exp2(sv[i] - m_new);
-        lsum = lsum * alpha +
-               (((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])));
+        for (int i = 0; i < 4 * TILES; i++)  // fp32: the scaling and the difference round once
+            p[i] = fast_exp2(F32 ? (sv[i] == -INFINITY ? sv[i] : fmaf(s[0][i & 3], scale_log2, -m_new))
+                                 : sv[i] - m_new);
+        float psum = (p[0] + p[1]) + (p[2] + p[3]);
+        if constexpr (TILES == 2) psum += (p[4] + p[5]) + (p[6] + p[7]);
+        lsum = lsum * alpha + psum;
         if (__builtin_amdgcn_ballot_w64(m_new > m) != 0) {
 #pragma unroll
             for (int nn = 0; nn < NV; nn++) acc[nn] *= alpha;
         }
         m = m_new;
-        // P^T as the B operand over the 32 tokens: lane (lg, lc) holds head lc at
-        // k-slots 8lg + j: j < 4 -> token 4lg + j (tile 0), j >= 4 -> 16 + 4lg + j - 4.
-        // Split hi + lo so the product keeps ~16 mantissa bits of P.
-        u32x4 PH, PL;
+        if constexpr (F32) {
+            // O^T += V^T P^T, one product per score register j and 16-dim block nn = 4i + e: B is
+            // the lane's p[j] (token 4lg + j, head lc), A the lane's V at that token, dim
+            // 64i + 4lc + e. The chunk is summed by itself and then added, so a long context's sum
+            // is a sum of chunk sums (fp32 rounding: relative error against 64 bits of 16 x 256-
+            // 2,048 tokens 2.7e-7 with one chain, the vector kernel 2.0e-7).
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t hi16 = pack2<T>(p[2 * i], p[2 * i + 1]);
-            PH[i] = hi16;
-            PL[i] = pack2<T>(p[2 * i] - lo_f32<T>(hi16), p[2 * i + 1] - hi_f32<T>(hi16));
-        }
-        // V^T as the A operand: lane (lg, lc) holds output dim (D / 16) lc + nn at the same
-        // k-slots, packed in-lane from its four V rows of each tile.
+            for (int nn = 0; nn < NV; nn++) {
+                f32x4 t = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int nn = 0; nn < NV; nn++) {
-            const int wd = nn >> 1;
-            u32x4 A;
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                if (nn & 1) {
-                    A[2 * t] = perm_hi16(va[t][0][wd], va[t][1][wd]);
-                    A[2 * t + 1] = perm_hi16(va[t][2][wd], va[t][3][wd]);
-                } else {
-                    A[2 * t] = perm_lo16(va[t][0][wd], va[t][1][wd]);
-                    A[2 * t + 1] = perm_lo16(va[t][2][wd], va[t][3][wd]);
-                }
+                for (int j = 0; j < 4; j++)
+                    t = mfma16x16x4_f32(__uint_as_float(va[nn >> 2][j][nn & 3]), p[j], t);
+                acc[nn] += t;
             }
-            acc[nn] = mfma16x16x32<T>(A, PH, acc[nn]);
-            acc[nn] = mfma16x16x32<T>(A, PL, acc[nn]);
+        } else {
+            // P^T as the B operand over the 32 tokens: lane (lg, lc) holds head lc at
+            // k-slots 8lg + j: j < 4 -> token 4lg + j (tile 0), j >= 4 -> 16 + 4lg + j - 4.
+            // Split hi + lo so the product keeps ~16 mantissa bits of P.
+            u32x4 PH, PL;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t hi16 = pack2<T>(p[2 * i], p[2 * i + 1]);
+                PH[i] = hi16;
+                PL[i] = pack2<T>(p[2 * i] - lo_f32<T>(hi16), p[2 * i + 1] - hi_f32<T>(hi16));
+            }
+            // V^T as the A operand: lane (lg, lc) holds output dim (D / 16) lc + nn at the same
+            // k-slots, packed in-lane from its four V rows of each tile.
+#pragma unroll
+            for (int nn = 0; nn < NV; nn++) {
+                const int wd = nn >> 1;
+                u32x4 A;
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    if (nn & 1) {
+                        A[2 * t] = perm_hi16(va[t][0][wd], va[t][1][wd]);
+                        A[2 * t + 1] = perm_hi16(va[t][2][wd], va[t][3][wd]);
+                    } else {
+                        A[2 * t] = perm_lo16(va[t][0][wd], va[t][1][wd]);
+                        A[2 * t + 1] = perm_lo16(va[t][2][wd], va[t][3][wd]);
+                    }
+                }
+                acc[nn] = mfma16x16x32<T>(A, PH, acc[nn]);
+                acc[nn] = mfma16x16x32<T>(A, PL, acc[nn]);
+            }
         }
     };
 
     // Piece epilogue from registers: lane (lg, lc) holds head lc, dims (D / 4) lg + NV r + nn
-    // (r < 4, nn < NV): D / 4 contiguous dims.
+    // (r < 4, nn < NV): D / 4 contiguous dims; fp32 pools: dims 64i + 16lg + 4r + e for nn = 4i + e.
     auto epilogue = [&](int b, int g, bool complete, bool first_piece) {
         lsum = sum_across_rows(lsum);
         // lg made opaque here, so the per-lane output addresses are formed at the store instead
@@ -475,11 +554,23 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
         if (lc < n_rep) {
             if (complete) {  // whole pair in this range: final output
                 const int64_t row = ws.rows ? (int64_t)ws.rows[b] : (int64_t)b;
-                TO* o = out + (row * num_heads + (int64_t)g * n_rep + lc) * D + (D / 4) * lgo;
+                TO* o = out + (row * num_heads + (int64_t)g * n_rep + lc) * D +
+                        (F32 ? 16 : D / 4) * lgo;
                 const float inv = 1.0f / lsum;
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    if constexpr (sizeof(TO) == 4) {
+                    if constexpr (F32) {
+#pragma unroll
+                        for (int h4 = 0; h4 < NV; h4 += 4) {
+                            const f32x4 v = f32x4{acc[h4][r] * inv, acc[h4 + 1][r] * inv,
+                                                  acc[h4 + 2][r] * inv, acc[h4 + 3][r] * inv};
+                            if constexpr (sizeof(TO) == 4)
+                                *reinterpret_cast<f32x4*>(o + 16 * h4 + 4 * r) = v;
+                            else
+                                *reinterpret_cast<u32x2*>(o + 16 * h4 + 4 * r) =
+                                    u32x2{pack2<TO>(v[0], v[1]), pack2<TO>(v[2], v[3])};
+                        }
+                    } else if constexpr (sizeof(TO) == 4) {
 #pragma unroll
                         for (int h4 = 0; h4 < NV; h4 += 4)
                             *reinterpret_cast<f32x4*>(o + NV * r + h4) =
@@ -498,12 +589,12 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
                 }
             } else {  // partial row for the merge kernel
                 const int64_t pidx = (2 * wgi + (first_piece ? 0 : 1)) * n_rep + lc;
-                float* o = ws.o + pidx * D + (D / 4) * lgo;
+                float* o = ws.o + pidx * D + (F32 ? 16 : D / 4) * lgo;
 #pragma unroll
                 for (int r = 0; r < 4; r++)
 #pragma unroll
                     for (int h4 = 0; h4 < NV; h4 += 4)
-                        *reinterpret_cast<f32x4*>(o + NV * r + h4) =
+                        *reinterpret_cast<f32x4*>(o + (F32 ? 16 * h4 + 4 * r : NV * r + h4)) =
                             f32x4{acc[h4][r], acc[h4 + 1][r], acc[h4 + 2][r], acc[h4 + 3][r]};
                 if (lg == 0) {
                     ws.ml[2 * pidx] = m;
@@ -601,7 +692,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
     int nx = cur.ce - cur.cb;
     bool has_nxt = nx < len;
     Seg nxt = cur;
-    Slots nxt_slots = cur_slots;
+    Slots nxt_slots{0, 0};  // (not a copy of cur_slots, which would wait for its load)
     if (has_nxt) {
         nxt = seg_at(nx);
         nxt_slots = seg_slots(nxt);
@@ -635,7 +726,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
             const bool in_cur = c + 1 < cur.ce;
             const int pg = in_cur ? cur.g : nxt.g;
             const Slots pslots = in_cur ? cur_slots : nxt_slots;
-            const int ptile = in_cur ? 2 * (c + 1 - cur.cb) : 0;
+            const int ptile = in_cur ? TILES * (c + 1 - cur.cb) : 0;
             load_chunk(pg, pslots, ptile, kn, vn);
         }
         compute_chunk(c, cur.tok_end, kc, vc);
@@ -675,7 +766,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
 
     using pf_on = std::integral_constant<bool, true>;
     using pf_off = std::integral_constant<bool, false>;
-    Ld ka[2][4], va[2][4], kb[2][4], vb[2][4];
+    Ld ka[NL][4], va[NL][4], kb[NL][4], vb[NL][4];
     load_chunk(cur.g, cur_slots, 0, ka, va);
     int remaining = len;  // chunks this wave computes; all but the last prefetch one
     for (; remaining > 2; remaining -= 2) {
@@ -719,7 +810,7 @@ __global__ __launch_bounds__(64 * DEC_MERGE_WAVES) void paged_decode_merge_kerne
         return;
     }
     const int g = h / n_rep, hh = h - g * n_rep;
-    const int64_t total = (int64_t)kv_heads * all, nwg = nwg_i;
+    const int64_t total = (int64_t)kv_heads * all, nwg = range_count(total, nwg_i);
     const int64_t s = (int64_t)kv_heads * before + (int64_t)g * nch;
     const int64_t e = s + nch;
     const bool narrow = ranges_narrow(total, nwg, ws.xcd_w);
@@ -732,18 +823,14 @@ __global__ __launch_bounds__(64 * DEC_MERGE_WAVES) void paged_decode_merge_kerne
     const int64_t l = narrow ? (int64_t)r32.owner((uint32_t)(e - 1)) : r64.owner(e - 1);
     const bool f_first = s == range_lo(f);
     if (f == l) return;  // finished inside one wave range
-    const int np = (int)(l - f + 1);  // ranges f..l; empty ones wrote nothing
+    const int np = (int)(l - f + 1);  // ranges f..l, none of them empty
 
     float M = -INFINITY, L = 0.0f, O[E];
 #pragma unroll
     for (int i = 0; i < E; i++) O[i] = 0.0f;
     const int fslot = (int)(f_first ? 2 * f : 2 * f + 1);  // the first piece always exists
-    // Wave ranges can be empty only when the smallest share, (32 - w) / 32 of the mean, is below
-    // one chunk; otherwise skip the range-bound divisions.
-    const bool dense = total * (32 - ws.xcd_w) >= 32 * nwg + 32;
-    auto piece_slot = [&](int64_t p) -> int {  // slot of piece p (< np), -1 for an empty range
+    auto piece_slot = [&](int64_t p) -> int {  // slot of piece p (< np)
         const int64_t ij = f + p;
-        if (!dense && range_lo(ij) == range_lo(ij + 1)) return -1;
         return (int)((ij == f && !f_first) ? 2 * ij + 1 : 2 * ij);
     };
     typedef typename std::conditional<E == 2, f32x2, float>::type RowV;
@@ -764,6 +851,7 @@ __global__ __launch_bounds__(64 * DEC_MERGE_WAVES) void paged_decode_merge_kerne
     for (int p0 = w_id * per; p0 < p_end; p0 += 64) {
         // The batch's first 8 pieces' rows are loaded before the (max, sum) reductions, which
         // they do not depend on (a missing piece reads the first piece's row, weight 0).
+        const int slot = p0 + lane < p_end ? piece_slot(p0 + lane) : -1;
         RowV v0[8];
         int s0[8];
 #pragma unroll
@@ -771,7 +859,6 @@ __global__ __launch_bounds__(64 * DEC_MERGE_WAVES) void paged_decode_merge_kerne
             s0[j] = p0 + j < p_end ? piece_slot(p0 + j) : -1;
             v0[j] = row(s0[j] >= 0 ? s0[j] : fslot);
         }
-        const int slot = p0 + lane < p_end ? piece_slot(p0 + lane) : -1;
         float mx = -INFINITY, lx = 0.0f;
         if (slot >= 0) {
             mx = ws.ml[2 * ((int64_t)slot * n_rep + hh)];
@@ -820,28 +907,42 @@ __global__ __launch_bounds__(64 * DEC_MERGE_WAVES) void paged_decode_merge_kerne
         for (int i = 0; i < E; i++) wO[w_id][i][lane] = O[i];
         __syncthreads();
         if (w_id != 0) return;
+        // all states are read together; slots past the last wave with pieces read its own
+        float mx[DEC_MERGE_WAVES], lx[DEC_MERGE_WAVES], ox[DEC_MERGE_WAVES][E];
         float Mt = M;
-        for (int x = 1; x < waves; x++) Mt = fmaxf(Mt, wM[x]);
+#pragma unroll
+        for (int x = 1; x < DEC_MERGE_WAVES; x++) {
+            const bool on = x < waves && x * per < np;
+            const int y = on ? x : 0;
+            mx[x] = on ? wM[y] : -INFINITY;
+            lx[x] = wL[y];
+#pragma unroll
+            for (int i = 0; i < E; i++) ox[x][i] = wO[y][i][lane];
+        }
+#pragma unroll
+        for (int x = 1; x < DEC_MERGE_WAVES; x++) Mt = fmaxf(Mt, mx[x]);
         const float f0 = fast_exp2(M - Mt);
         L *= f0;
 #pragma unroll
         for (int i = 0; i < E; i++) O[i] *= f0;
-        for (int x = 1; x < waves; x++) {
-            if (x * per >= np) break;  // no pieces there
-            const float f = fast_exp2(wM[x] - Mt);
-            L += wL[x] * f;
 #pragma unroll
-            for (int i = 0; i < E; i++) O[i] += wO[x][i][lane] * f;
+        for (int x = 1; x < DEC_MERGE_WAVES; x++) {
+            if (x < waves && x * per < np) {
+                const float f = fast_exp2(mx[x] - Mt);
+                L += lx[x] * f;
+#pragma unroll
+                for (int i = 0; i < E; i++) O[i] += ox[x][i] * f;
+            }
         }
     }
 #pragma unroll
     for (int i = 0; i < E; i++) o[i] = from_f32<TO>(O[i] / L);
 }
 
-// Waves per merge workgroup: about eight pieces (one memory round trip) each, for the mean number
-// of pieces per pair and twice that on the longest contexts.
-static int decode_merge_waves(int nwg, int batch, int kv_heads) {
-    const int64_t pieces = 2 * (int64_t)nwg / ((int64_t)batch * kv_heads);
+// Waves per merge workgroup: about eight pieces (one memory round trip) each, for twice the mean
+// number of pieces per pair (longer contexts than the mean have more).
+static int decode_merge_waves(int grid, int batch, int kv_heads) {
+    const int64_t pieces = 2 * (int64_t)grid / ((int64_t)batch * kv_heads);
     int waves = 1;
     while (waves < DEC_MERGE_WAVES && 8 * waves < pieces) waves *= 2;
     return waves;
@@ -859,18 +960,23 @@ static int launch_decode_mfma_d(void* out, const void* q, const void* k_pool, co
         set_error("paged_decode: the fused KV write needs 16-token pages");
         return FLOUR_ERR_UNSUPPORTED;
     }
-    auto kern = block_size == 16 ? (fuse ? paged_decode_mfma_kernel<T, TO, true, D, true>
-                                         : paged_decode_mfma_kernel<T, TO, true, D, false>)
+    auto kern = block_size == 16 ? paged_decode_mfma_kernel<T, TO, true, D, false>
                                  : paged_decode_mfma_kernel<T, TO, false, D, false>;
-    kern<<<dim3(nwg), dim3(64), lds, stream>>>(
+    if constexpr (!std::is_same<T, float>::value)  // (fp32 pools take no fused write)
+        if (fuse) kern = paged_decode_mfma_kernel<T, TO, true, D, true>;
+    // no more waves than ranges (range_count) for contexts of max_ctx
+    const int64_t chunk = dec_chunk(sizeof(T));
+    const int64_t half = (int64_t)batch * kv_heads * ((max_ctx + chunk - 1) / chunk) / 2;
+    const int grid = (int)(half < 1 ? 1 : half < nwg ? half : nwg);
+    kern<<<dim3(grid), dim3(64), lds, stream>>>(
         static_cast<TO*>(out), static_cast<const T*>(q), static_cast<const T*>(k_pool),
         static_cast<const T*>(v_pool), bt, max_blocks, ctx_lens, batch, num_heads, kv_heads, n_rep,
         block_size, num_slots, max_ctx, scale * LOG2E, ws);
     int rc = check_hip(hipGetLastError(), "paged_decode launch");
     if (rc != FLOUR_OK) return rc;
-    const int mw = decode_merge_waves(nwg, batch, kv_heads);
+    const int mw = decode_merge_waves(grid, batch, kv_heads);
     paged_decode_merge_kernel<TO, D><<<dim3(num_heads, batch), dim3(64 * mw), 0, stream>>>(
-        static_cast<TO*>(out), batch, num_heads, kv_heads, n_rep, nwg, ws);
+        static_cast<TO*>(out), batch, num_heads, kv_heads, n_rep, grid, ws);
     return check_hip(hipGetLastError(), "paged_decode merge launch");
 }
 
@@ -925,7 +1031,7 @@ extern "C" int flour_hip_paged_decode_workspace_size(int batch, int num_heads, i
         set_error("paged_decode_workspace_size: bad arguments");
         return FLOUR_ERR_INVALID_ARGUMENT;
     }
-    *bytes = decode_ws_bytes(decode_workgroups(), num_heads / kv_heads, head_dim, batch);
+    *bytes = decode_ws_bytes(decode_workgroups(FLOUR_DTYPE_F32), num_heads / kv_heads, head_dim, batch);
     return FLOUR_OK;
 }
 
@@ -1026,6 +1132,29 @@ bool decode_mfma_supported(int dtype, int head_dim, int block_size, int n_rep, i
            ((uintptr_t)k_pool % 16 == 0) && ((uintptr_t)v_pool % 16 == 0);
 }
 
+// Whether an fp32 batch runs split over the chip on the matrix cores (with this workspace) rather
+// than on the vector kernel, which needs no workspace but gives each (sequence, kv head) one
+// workgroup.
+static bool decode_f32_split(int head_dim, int block_size, int n_rep, int batch, int num_heads,
+                             int64_t num_slots, int max_context_len, const void* q,
+                             const void* k_pool, const void* v_pool, bool ws_ok) {
+    if (!ws_ok || (head_dim != 128 && head_dim != 64) || block_size % 16 != 0 || n_rep > 16 ||
+        batch > DEC_MAX_BATCH || num_heads > 65535 ||
+        num_slots * head_dim * 4 > (int64_t)0x7fffffff ||
+        (((uintptr_t)q | (uintptr_t)k_pool | (uintptr_t)v_pool) & 15) != 0)
+        return false;
+    // The vector kernel's time goes with a workgroup's kv length x queries (n_rep, as a power of
+    // two) x head_dim; a split step takes ~9 us and its bytes. Vector / split in us: 1 x 256 tokens of
+    // 32 / 8 heads of 128 14.5 / 10.3 (64 tokens: 7.4 / 9.8), 14 / 2 heads of 64 13.4 / 8.8 (64: 8.3 /
+    // 8.4), 16 / 16 of 128 at 1,024 18.3 / 11.8 (256: 7.7 / 10.2), 8 / 8 of 64 at 2,048 19.9 / 10.0
+    // (512: 8.1 / 9.0). At n_rep 1 with one full round of workgroups the vector kernel is better
+    // for as long again: 16 x 8 / 8 heads of 64 at 2,048 23.8 / 26.3, at 8,192 102 / 79.
+    int64_t work = (int64_t)max_context_len * head_dim;
+    for (int nq = 1; nq < n_rep && nq < 8; nq *= 2) work *= 2;
+    const int64_t pairs = (int64_t)batch * num_heads / n_rep;
+    return work >= (n_rep == 1 && pairs >= 128 && pairs <= 256 ? 262144 : 131072);
+}
+
 static int paged_decode_impl(void* out, int out_dtype, const void* q, const void* k_pool,
                              const void* v_pool, const int32_t* block_tables,
                              int max_blocks_per_seq, const int32_t* context_lens, int batch,
@@ -1060,7 +1189,16 @@ static int paged_decode_impl(void* out, int out_dtype, const void* q, const void
         set_error("paged_decode: row indices and the fused KV write need the matrix-core path");
         return FLOUR_ERR_UNSUPPORTED;
     }
-    if (!mfma) {
+    const int nwg = decode_workgroups(dtype);
+    const size_t need = decode_ws_bytes(nwg, n_rep, head_dim, batch);
+    const bool ws_ok = ws_from_scratch ? need <= DEC_SCRATCH_BYTES
+                                       : workspace && workspace_bytes >= need &&
+                                             ((uintptr_t)workspace % 256) == 0;
+    const bool f32_split =
+        dtype == FLOUR_DTYPE_F32 && decode_f32_split(head_dim, block_size, n_rep, batch, num_heads,
+                                                     num_slots, max_context_len, q, k_pool, v_pool,
+                                                     ws_ok);
+    if (!mfma && !f32_split) {
         // one query row per sequence: cu_seqlens == nullptr
         const int64_t qs = (int64_t)num_heads * head_dim;
         if (simt_supported(dtype, head_dim, q, qs, head_dim, k_pool, v_pool))
@@ -1074,8 +1212,6 @@ static int paged_decode_impl(void* out, int out_dtype, const void* q, const void
                                    batch, num_heads, n_rep, head_dim, block_size, num_slots,
                                    max_context_len, scale, s);
     }
-    const int nwg = decode_workgroups();
-    const size_t need = decode_ws_bytes(nwg, n_rep, head_dim, batch);
     if (ws_from_scratch) {
         if (need > DEC_SCRATCH_BYTES) {
             set_error("paged_decode_noalloc: this call needs %zu bytes of split-context workspace, "
@@ -1088,7 +1224,7 @@ static int paged_decode_impl(void* out, int out_dtype, const void* q, const void
         if (rc != FLOUR_OK) return rc;
         workspace_bytes = DEC_SCRATCH_BYTES;
     }
-    if (!workspace || workspace_bytes < need || ((uintptr_t)workspace % 256) != 0) {
+    if (!ws_ok) {
         set_error("paged_decode: workspace of %zu bytes (256-byte aligned) required, got %zu "
                   "at %p",
                   need, workspace_bytes, workspace);
@@ -1127,6 +1263,7 @@ static int paged_decode_impl(void* out, int out_dtype, const void* q, const void
                                             max_context_len, scale, nwg, ws, s);                \
     } while (0)
     if (dtype == FLOUR_DTYPE_BF16) FLOUR_DEC(bf16_t);
+    if (dtype == FLOUR_DTYPE_F32) FLOUR_DEC(float);
     FLOUR_DEC(f16_t);
 #undef FLOUR_DEC
 }

@@ -72,6 +72,54 @@ def test_decode_fp32_small_shapes(device, H, G, D, bs, ctx):
     assert max_abs <= 1e-5
 
 
+@pytest.mark.parametrize("H,G,D,bs,ctx", [
+    (32, 8, 128, 16, [4096, 1, 15, 16, 17, 0, 33, 500]),  # partial tiles, an empty context
+    (16, 16, 128, 32, [3000, 31]),                        # n_rep 1, 32-token pages
+    (14, 2, 64, 16, [2049]),                              # n_rep 7, one sequence: many pieces
+    (16, 1, 64, 48, [2500, 7, 700]),                      # n_rep 16, 48-token pages
+    (8, 8, 64, 16, [4097] * 3 + list(range(1, 70))),      # more than 64 sequences
+])
+def test_decode_fp32_split(device, H, G, D, bs, ctx):
+    """fp32 steps long enough to be split over the chip on the fp32 matrix cores: against the
+    oracle (products and sums in fp32: the bound of the other fp32 paths), for every output type,
+    and against the vector kernel, which a call without a workspace takes."""
+    from flour_amd import _lib
+    c = make_decode(len(ctx), H, G, D, bs, (1, 1), dtype=torch.float32, seed=H * D + bs,
+                    device=device, context_lens=ctx)
+    vec = torch.empty_like(c.q)
+    p = ops._ptr
+    _lib.check(_lib.lib().flour_hip_paged_decode(
+        p(vec), 0, p(c.q), p(c.k_pool), p(c.v_pool), p(c.block_tables), c.block_tables.shape[1],
+        p(c.context_lens), len(ctx), H, G, D, bs, c.k_pool.shape[1], c.max_context_len, c.scale, 0,
+        None, 0, ops._stream()))
+    torch.cuda.synchronize()
+    assert errors(to_np(vec), oracle_decode(c))[0] <= 1e-5
+    # rows past the contexts hold garbage that must not leak in
+    used = torch.zeros(c.k_pool.shape[1], dtype=torch.bool)
+    for s, n in enumerate(ctx):
+        j = torch.arange(n)
+        used[c.block_tables[s].cpu()[j // bs].long() * bs + j % bs] = True
+    c.k_pool[:, ~used.to(device)] = float("nan")
+    c.v_pool[:, ~used.to(device)] = float("inf")
+    ref = oracle_decode(c)
+    got = run(c)
+    max_abs, _ = errors(to_np(got), ref)
+    print(f"fp32 split max_abs={max_abs:.3e}", flush=True)
+    assert max_abs <= 1e-5
+    for dt in (torch.bfloat16, torch.float16):  # the fp32 result, rounded once
+        assert torch.equal(run(c, dt), got.to(dt))
+
+
+@pytest.mark.parametrize("ctx", [[1], [33], [65, 2], [100], [1000], [5000], [40] * 65])
+def test_decode_few_chunks(device, ctx):
+    """Chunk lists shorter than the grid (at least two chunks a range) and merges split over
+    several waves."""
+    for H, G, D in ((8, 1, 128), (32, 8, 128), (14, 2, 64)):
+        c = make_decode(len(ctx), H, G, D, 16, (1, 1), dtype=torch.bfloat16, seed=len(ctx) + H,
+                        device=device, context_lens=ctx)
+        check_bf16(c, f"few chunks {ctx[:2]}")
+
+
 @pytest.mark.parametrize("H,G,ctx", [
     (32, 8, [1, 2, 15, 16, 17, 31, 63, 64, 65, 100]),   # partial tiles, one split
     (8, 8, [1000, 513, 2049]),                          # n_rep 1, several splits
