@@ -241,6 +241,296 @@ __global__ __launch_bounds__(f32m_waves(D) * 64) void prefill_f32_mfma_kernel(
     }
 }
 
+// ---- Larger batches. An item is (kv head, group of HW query heads, sequence, 32 (4 / HW) query
+// rows), HW = 4, 2 or 1, for a workgroup of eight waves: waves w and w + 4, which share a SIMD, own
+// the same 32 rows of one head and take alternate 32-position tiles; their states are folded at
+// the end. K / V rows go straight into LDS, once for all eight waves (double-buffered, one barrier
+// per step of 64 positions, 128 at D 64, loads one step ahead and block ids two), where the kernel
+// above has every wave gather its own from L2 with nothing in flight under its products. Bound by
+// the fp32 matrix cores: a wave's tile is D products of 64 cycles.
+//  * One workgroup per CU takes items longest first, as a snake over the list: left to the
+//    dispatcher, workgroups of this size fill the CUs in a fixed rotation and a ragged batch waits
+//    for the unluckiest (8 x U[300, 1,024] rows, 32 / 8 heads of 128: 461 us, dealt 352).
+//  * The first four waves run at raised priority and a wave keeps two chains of products going, so
+//    that a SIMD's second wave has its products left for the time of the first's softmax.
+//  * S^T as above, the 16-byte chunk c of K row r at chunk c ^ (r % 16) (conflict-free reads).
+//  * O^T tile t holds dims 32 t .. 32 t + 31: its A operand is V[position][32 t + lane % 32], a
+//    4-byte read of a V row, so V needs no transpose.
+//  * fp32 sums are kept short (chains of 32 products for a score, of the tile's 32 positions for
+//    an output, then sums of those): error against 64 bits 1.4-2.4e-7 over 25 batches, where the
+//    kernel above has 2.2-5.1e-7.
+// Against the kernel above: 8 x U[256, 1,024] rows, 32 / 8 heads of 128, 429 -> 346 us (82
+// TFLOP/s); 16 x 512 552 -> 414; 1 x 4,096 1,327 -> 1,181 (116); 32 x U[256, 400], 14 / 2 heads of
+// 64, 153 -> 112.
+static constexpr int F32T_SPLIT = 2;  // waves per (head, row block)
+static constexpr int F32T_WAVES = 4 * F32T_SPLIT;
+static constexpr uint32_t F32T_OOR = 0x80000000u;  // buffer offset past any pool: loads read 0
+template <int D, bool BS16>
+__global__ __launch_bounds__(F32T_WAVES * 64, 2) void prefill_f32_tile_kernel(
+    void* __restrict__ out, int out_dtype, int64_t o_st, int64_t o_sh,
+    const float* __restrict__ q, int64_t q_st, int64_t q_sh, const float* __restrict__ k_pool,
+    const float* __restrict__ v_pool, const int32_t* __restrict__ cu_seqlens_q,
+    const int32_t* __restrict__ kv_lens, const int32_t* __restrict__ block_tables, int max_blocks,
+    int num_seqs, int kv_heads, int n_rep, int hw, int block_size, int num_slots, int n_qt,
+    float scale_log2) {
+    constexpr int DH = D / 2, DT = D / 32;
+    constexpr int SUB = 128 / D;              // 32-position tiles per wave and step
+    constexpr int KT = F32M_KT * F32T_SPLIT * SUB;  // positions per step
+    constexpr int CPR = D / 4;                // 16-byte chunks per row
+    constexpr int RPL = 64 / CPR;             // rows per wave load of 1 KB
+    constexpr int NP = KT / (RPL * F32T_WAVES);  // loads per wave, step and pool (4 at D 128)
+    constexpr int NS = 16 * DT + 2;           // a lane's state: O^T registers, max, sum
+    __shared__ __attribute__((aligned(16))) float lds[4 * KT * D];
+    static_assert(4 * (F32T_SPLIT - 1) * NS * 64 <= 4 * KT * D, "the states fit the tiles");
+    auto kt = [&](int buf) { return lds + buf * KT * D; };
+    auto vt = [&](int buf) { return lds + (2 + buf) * KT * D; };
+
+    const int groups = (n_rep + hw - 1) / hw, per_row = kv_heads * groups;
+    const int rows = F32M_QT * (4 / hw);  // query rows of an item
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int r = lane & 31, h = lane >> 5;
+    const int wq = w & 3, ks = w >> 2;  // (head, row block), part of each step
+    const int max_phys = num_slots / block_size - 1;
+    const uint32_t head_bytes = (uint32_t)num_slots * D * 4u;
+    const int G = gridDim.x;
+
+    // The items, longest first: tile index (level) by decreasing level, then sequence, then head
+    // group. Every wave walks the levels by itself with one sequence per lane.
+    const int my_c0 = cu_seqlens_q[min(lane, num_seqs)];
+    const int my_rows = lane < num_seqs ? cu_seqlens_q[lane + 1] - my_c0 : 0;
+    const int my_kv = lane < num_seqs ? min(kv_lens[lane], max_blocks * block_size) : 0;
+    const int my_tiles = my_rows > 0 ? (my_rows + rows - 1) / rows : 0;
+    int level = n_qt - 1, base = 0;  // items of the levels above `level`
+    uint64_t there = __ballot(my_tiles > level);
+    if (ks == 0) __builtin_amdgcn_s_setprio(1);
+
+    for (int round = 0;; round++) {
+        // a snake over the list: even rounds in workgroup order, odd ones reversed
+        const int idx = round * G + ((round & 1) ? G - 1 - (int)blockIdx.x : (int)blockIdx.x);
+        while (level >= 0 && idx >= base + per_row * __popcll(there)) {
+            base += per_row * __popcll(there);
+            level--;
+            there = __ballot(my_tiles > level);
+        }
+        if (level < 0) break;  // past the list, and so is every later round's index
+        const int rank = (idx - base) / per_row, x = idx - base - rank * per_row;
+        const uint64_t nth =
+            __ballot(((there >> lane) & 1) && __popcll(there & ((1ull << lane) - 1)) == rank);
+        const int s = __ffsll((unsigned long long)nth) - 1;
+        const int qt = level;
+        const int kvh = x / groups, h0 = (x - kvh * groups) * hw;
+        const int c0 = __builtin_amdgcn_readlane(my_c0, s);
+        const int q_len = __builtin_amdgcn_readlane(my_rows, s);
+        const int kv_len = __builtin_amdgcn_readlane(my_kv, s);
+        const int off = kv_len - q_len;  // row i sees positions j <= off + i
+        const bool reads = kv_len >= q_len;
+        const int kv_end = reads ? off + min(qt * rows + rows, q_len) : 0;  // the item's range
+        const int hl = h0 + wq % hw;
+        const int i0 = qt * rows + F32M_QT * (wq / hw);  // the wave's first row
+        const bool active = hl < n_rep && i0 < q_len;    // uniform over the wave
+        const int i = i0 + r;
+        const int head = kvh * n_rep + min(hl, n_rep - 1);
+        const int lim = (active && i < q_len && reads) ? off + i : -1;
+        const int w_end = active && reads ? off + min(i0 + F32M_QT, q_len) : 0;  // the wave's range
+        const int w_full = off + i0;  // positions up to here are visible to every row of the wave
+        const int32_t* bt = block_tables + (int64_t)s * max_blocks;
+        const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(k_pool + (int64_t)kvh * num_slots * D), (short)0, (int)head_bytes, BUF_DWORD3);
+        const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(v_pool + (int64_t)kvh * num_slots * D), (short)0, (int)head_bytes, BUF_DWORD3);
+
+        float qv[DH];
+        {
+            const float* qp =
+                q + (int64_t)(c0 + min(i, q_len - 1)) * q_st + (int64_t)head * q_sh + DH * h;
+#pragma unroll
+            for (int y = 0; y < DH / 4; y++) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(qp + 4 * y);
+#pragma unroll
+                for (int e = 0; e < 4; e++) qv[4 * y + e] = v[e] * scale_log2;
+            }
+        }
+
+        // Staging, straight into LDS: load p of wave w fills rows srow + RPL F32T_WAVES p of the
+        // step, lane l chunk l % CPR of row l / CPR. A K row's chunk c sits at chunk c ^ (row % 16)
+        // (conflict-free fragment reads), so the lane reads that chunk of the row; V as it is.
+        const int lrow = lane / CPR, lchunk = lane % CPR;
+        const int srow = RPL * w + lrow;
+        auto load_ids = [&](int kv0, int* ids) __attribute__((always_inline)) {
+#pragma unroll
+            for (int p = 0; p < NP; p++) {
+                const int j = min(kv0 + srow + RPL * F32T_WAVES * p, max(kv_end - 1, 0));
+                ids[p] = bt[BS16 ? j >> 4 : j / block_size];
+            }
+        };
+        auto load_tile = [&](int kv0, const int* ids, int buf) __attribute__((always_inline)) {
+#pragma unroll
+            for (int p = 0; p < NP; p++) {
+                const int row = srow + RPL * F32T_WAVES * p, j = kv0 + row;
+                const int in = BS16 ? j & 15 : j % block_size;
+                const int phys = min(max(ids[p], 0), max_phys);  // a bad block id stays in the pool
+                const uint32_t at = (uint32_t)(phys * block_size + in) * (uint32_t)(4 * D);
+                const bool there = j < kv_end;  // rows past the range read zeros (masked anyway)
+                const uint32_t dst = (uint32_t)(RPL * (w + F32T_WAVES * p)) * (uint32_t)(4 * D);
+                dma_b128(there ? at + 16u * (uint32_t)(lchunk ^ (row & 15)) : F32T_OOR, k_rsrc,
+                         lds_byte_addr(kt(buf)) + dst, 0u);
+                dma_b128(there ? at + 16u * (uint32_t)lchunk : F32T_OOR, v_rsrc,
+                         lds_byte_addr(vt(buf)) + dst, 0u);
+            }
+        };
+
+        float m = -INFINITY, l = 0.0f;
+        f32x16 o[DT];
+#pragma unroll
+        for (int t = 0; t < DT; t++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) o[t][e] = 0.0f;
+
+        const int n_st = (kv_end + KT - 1) / KT;
+        int ids[NP];
+        load_ids(0, ids);
+        __syncthreads();  // the last item's states are read
+        if (n_st > 0) {
+            load_tile(0, ids, 0);
+            load_ids(KT, ids);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        for (int st = 0; st < n_st; st++) {
+            const int buf = st & 1;
+            if (st + 1 < n_st) {
+                load_tile((st + 1) * KT, ids, buf ^ 1);
+                load_ids((st + 2) * KT, ids);
+            }
+#pragma unroll
+            for (int u = 0; u < SUB; u++) {
+                const int row0 = F32M_KT * (ks + F32T_SPLIT * u);  // the wave's tile in the step
+                const int kv0 = st * KT + row0;
+                if (kv0 >= w_end) continue;  // uniform over the wave
+                const float* kr = kt(buf) + (row0 + r) * D;
+                f32x16 sc;
+                // two chains of 32 products (16 steps of k = 2) at a time: independent products
+                // keep the matrix core busy from one wave
+#pragma unroll
+                for (int c = 0; c < DH / 32; c++) {
+                    f32x16 pa, pb;
+#pragma unroll
+                    for (int e = 0; e < 16; e++) pa[e] = pb[e] = 0.0f;
+#pragma unroll
+                    for (int y = 0; y < 4; y++) {
+                        // chunk DH / 4 h + 8c + y (+ 4) of the row
+                        const int ca = (DH / 4) * h + 8 * c + y;
+                        const f32x4 ka = *reinterpret_cast<const f32x4*>(kr + 4 * (ca ^ (r & 15)));
+                        const f32x4 kb = *reinterpret_cast<const f32x4*>(kr + 4 * ((ca + 4) ^ (r & 15)));
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            pa = mfma32x32x2_f32(ka[e], qv[32 * c + 4 * y + e], pa);
+                            pb = mfma32x32x2_f32(kb[e], qv[32 * c + 16 + 4 * y + e], pb);
+                        }
+                    }
+                    if (c == 0)
+                        sc = pa + pb;
+                    else
+                        sc += pa + pb;
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (kv0 + F32M_KT - 1 > w_full) {  // the tile crosses some row's limit
+#pragma unroll
+                    for (int e = 0; e < 16; e++)
+                        if (kv0 + 8 * (e >> 2) + 4 * h + (e & 3) > lim) sc[e] = -INFINITY;
+                }
+                float tm = sc[0];
+#pragma unroll
+                for (int e = 1; e < 16; e++) tm = fmaxf(tm, sc[e]);
+                tm = max_across_halves(tm);
+                const float m_new = fmaxf(m, tm);
+                const float mu = m_new == -INFINITY ? 0.0f : m_new;  // nothing visible: all p = 0
+                const float alpha = fast_exp2(m - mu);
+                m = m_new;
+                float ps = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    sc[e] = fast_exp2(sc[e] - mu);
+                    ps += sc[e];
+                }
+                l = l * alpha + ps;
+                const float* vr = vt(buf) + (row0 + 4 * h) * D + r;
+#pragma unroll
+                for (int t = 0; t < DT; t += 2) {
+                    f32x16 pa, pb;
+#pragma unroll
+                    for (int e = 0; e < 16; e++) pa[e] = pb[e] = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < 16; e++) {
+                        const float* v = vr + (8 * (e >> 2) + (e & 3)) * D + 32 * t;
+                        pa = mfma32x32x2_f32(v[0], sc[e], pa);
+                        pb = mfma32x32x2_f32(v[32], sc[e], pb);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 16; e++) o[t][e] = fmaf(o[t][e], alpha, pa[e]);
+#pragma unroll
+                    for (int e = 0; e < 16; e++) o[t + 1][e] = fmaf(o[t + 1][e], alpha, pb[e]);
+                }
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the next step's rows are in LDS
+            __syncthreads();
+        }
+        l = sum_across_halves(l);
+        // fold the two waves' states (the last step's barrier is behind every read of the tiles)
+        if (ks) {
+            float* dst = lds + wq * NS * 64 + lane;
+#pragma unroll
+            for (int t = 0; t < DT; t++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) dst[(16 * t + e) * 64] = o[t][e];
+            dst[16 * DT * 64] = m;
+            dst[(16 * DT + 1) * 64] = l;
+        }
+        __syncthreads();
+        if (!ks && active && i < q_len) {
+            const float* src = lds + wq * NS * 64 + lane;
+            const float mb = src[16 * DT * 64], lb = src[(16 * DT + 1) * 64];
+            const float mm = fmaxf(m, mb);
+            const float mz = mm == -INFINITY ? 0.0f : mm;
+            const float fa = fast_exp2(m - mz), fb = fast_exp2(mb - mz);
+            l = l * fa + lb * fb;
+            const float inv = l > 0.0f ? 1.0f / l : 0.0f;  // no visible position: a zero row
+            const int64_t obase = (int64_t)(c0 + i) * o_st + (int64_t)head * o_sh + 4 * h;
+#pragma unroll
+            for (int t = 0; t < DT; t++)
+#pragma unroll
+                for (int e = 0; e < 16; e += 4) {
+                    float v[4];
+#pragma unroll
+                    for (int y = 0; y < 4; y++)
+                        v[y] = (o[t][e + y] * fa + src[(16 * t + e + y) * 64] * fb) * inv;
+                    store_run<4>(out, out_dtype, obase + 32 * t + 2 * e, v);
+                }
+        }
+    }
+}
+
+// Query heads per item of the tile kernel: 4 or 2 where at most one wave in eight is left without
+// a head, else 1.
+static int f32_tile_heads(int n_rep) {
+    if (n_rep % 4 == 0 || (n_rep % 4 == 3 && n_rep > 3)) return 4;
+    return n_rep % 2 == 0 ? 2 : 1;
+}
+
+static int device_cus_f32() {
+    static int cached[64] = {0};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    if (cached[dev] == 0) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+            n <= 0)
+            n = 256;
+        cached[dev] = n;
+    }
+    return cached[dev];
+}
+
 static int g_prefill_f32_mfma = 1;  // a test / tuning switch
 
 bool prefill_f32_mfma_supported(int dtype, int head_dim, int num_seqs, int max_seqlen_q,
@@ -257,13 +547,39 @@ int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh
                             int64_t q_st, int64_t q_sh, const void* k_pool, const void* v_pool,
                             const int32_t* cu_seqlens_q, const int32_t* q_rows,
                             const int32_t* kv_lens, const int32_t* block_tables, int max_blocks,
-                            int num_seqs, int max_seqlen_q, int num_heads, int n_rep,
+                            int num_seqs, int max_seqlen_q, int total_q, int num_heads, int n_rep,
                             int head_dim, int block_size, int64_t num_slots, float scale,
                             hipStream_t stream) {
     const int n_qt = (max_seqlen_q + F32M_QT - 1) / F32M_QT;
     if (n_qt == 0 || num_seqs == 0) return FLOUR_OK;
     const dim3 grid((unsigned)num_heads, (unsigned)num_seqs, (unsigned)n_qt);
     const float sl2 = scale * 1.4426950408889634f;
+    // The tile kernel from two full-tile items per CU on (item tiles counted from the batch's rows):
+    // with fewer, an item's chain of steps bounds it, which the other kernel splits over 4 or 8
+    // waves. Measured, other / tile in us: 32 / 8 heads of 128, 1 x 1,024 rows (1 item per CU) 120 /
+    // 157, 2 x 1,024 203 / 168; 8 / 8 of 64, 1 x 1,024 (1/4) 29 / 77, 8 x 1,024 (2) 123 / 102; 16 /
+    // 16 of 128, 4 x U[512, 1,024] (1.5) 130 / 136; 14 / 2 of 64, 8 x U[256, 1,024] (2.5) 113 / 114.
+    // Its item list holds up to 64 sequences, its loads 32-bit offsets.
+    const int hw = f32_tile_heads(n_rep), kv_heads = num_heads / n_rep;
+    const int rows = F32M_QT * (4 / hw);
+    const int64_t per_row = (int64_t)kv_heads * ((n_rep + hw - 1) / hw);
+    const int64_t cus = device_cus_f32();
+    const bool tiled = !q_rows && num_seqs <= 64 && num_slots * head_dim * 4 <= 0x7fffffff &&
+                       per_row * (total_q / rows) >= 2 * cus &&
+                       per_row * num_seqs * ((int64_t)max_seqlen_q / rows + 1) <= 0x3fffffff;
+    if (tiled) {
+        const int nt = (max_seqlen_q + rows - 1) / rows;
+        auto kern = head_dim == 64 ? (block_size == 16 ? prefill_f32_tile_kernel<64, true>
+                                                       : prefill_f32_tile_kernel<64, false>)
+                                   : (block_size == 16 ? prefill_f32_tile_kernel<128, true>
+                                                       : prefill_f32_tile_kernel<128, false>);
+        kern<<<dim3((unsigned)cus), dim3(F32T_WAVES * 64), 0, stream>>>(
+            out, out_dtype, o_st, o_sh, static_cast<const float*>(q), q_st, q_sh,
+            static_cast<const float*>(k_pool), static_cast<const float*>(v_pool), cu_seqlens_q,
+            kv_lens, block_tables, max_blocks, num_seqs, kv_heads, n_rep, hw, block_size,
+            (int)num_slots, nt, sl2);
+        return check_hip(hipGetLastError(), "varlen_prefill (fp32 matrix cores) launch");
+    }
 #define FLOUR_F32M(D)                                                                            \
     prefill_f32_mfma_kernel<D><<<grid, dim3(f32m_waves(D) * 64), 0, stream>>>(                   \
         out, out_dtype, o_st, o_sh, static_cast<const float*>(q), q_st, q_sh,                    \

@@ -146,6 +146,27 @@ __device__ __forceinline__ f32x16 mfma32x32x16<f16_t>(u32x4 a, u32x4 b, f32x16 c
 static constexpr int BUF_DWORD3 = 0x00020000;
 static constexpr int BUF_NT = 2;
 
+// 64 lanes x 16 bytes from a raw buffer straight into LDS: lane L's bytes come from
+// rsrc.base + soff + voff and land at LDS byte lds + 16 L; lanes past the buffer's size write
+// zeros. Issued from inline asm so that the compiler's wait-count tracking, which knows nothing
+// of these loads, adds no waits for them to the LDS reads; every wait for them is explicit.
+// M0 (the LDS destination) is written here. The AMDGPU backend treats M0 as a reserved
+// register and ignores it in clobber lists; none of its own code in these kernels reads M0 (the
+// generated ISA has no M0 reader other than these loads), so no compiler value can be
+// overwritten. The s_nop 0 between the M0 write and the load is the wait state a vector memory
+// instruction that reads M0 needs after an SALU write of M0 (the hardware does not interlock
+// it, and the compiler's hazard tracking does not look inside inline asm).
+__device__ __forceinline__ void dma_b128(uint32_t voff, __amdgpu_buffer_rsrc_t rsrc, uint32_t lds,
+                                         uint32_t soff) {
+    const uint32_t l = __builtin_amdgcn_readfirstlane(lds);
+    const uint32_t so = __builtin_amdgcn_readfirstlane(soff);
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds"
+                 :: "v"(voff), "s"(rsrc), "s"(l), "s"(so) : "memory");
+}
+__device__ __forceinline__ uint32_t lds_byte_addr(const void* p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+
 // ------------------------------------------------------------------ misc device helpers
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 

@@ -52,7 +52,7 @@ int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh
                             int64_t q_st, int64_t q_sh, const void* k_pool, const void* v_pool,
                             const int32_t* cu_seqlens_q, const int32_t* q_rows,
                             const int32_t* kv_lens, const int32_t* block_tables, int max_blocks,
-                            int num_seqs, int max_seqlen_q, int num_heads, int n_rep,
+                            int num_seqs, int max_seqlen_q, int total_q, int num_heads, int n_rep,
                             int head_dim, int block_size, int64_t num_slots, float scale,
                             hipStream_t stream);
 bool simt_supported(int dtype, int head_dim, const void* q, int64_t q_st, int64_t q_sh,
@@ -143,23 +143,6 @@ static constexpr uint32_t PF_OOR = 0x80000000u;  // buffer offset past any pool:
 // attention launch.
 static constexpr int PF_VPAGE_BYTES = 16 * PF_D * 2;
 
-// 64 lanes x 16 bytes from a raw buffer straight into LDS: lane L's bytes come from
-// rsrc.base + soff + voff and land at LDS byte lds + 16 L; lanes past the buffer's size write
-// zeros. Issued from inline asm so that the compiler's wait-count tracking, which knows nothing
-// of these loads, adds no waits for them to the LDS reads; every wait for them is explicit.
-// M0 (the LDS destination) is written here. The AMDGPU backend treats M0 as a reserved
-// register and ignores it in clobber lists; none of its own code in these kernels reads M0 (the
-// generated ISA has no M0 reader other than these loads), so no compiler value can be
-// overwritten. The s_nop 0 between the M0 write and the load is the wait state a vector memory
-// instruction that reads M0 needs after an SALU write of M0 (the hardware does not interlock
-// it, and the compiler's hazard tracking does not look inside inline asm).
-__device__ __forceinline__ void dma_b128(uint32_t voff, __amdgpu_buffer_rsrc_t rsrc, uint32_t lds,
-                                         uint32_t soff) {
-    const uint32_t l = __builtin_amdgcn_readfirstlane(lds);
-    const uint32_t so = __builtin_amdgcn_readfirstlane(soff);
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds"
-                 :: "v"(voff), "s"(rsrc), "s"(l), "s"(so) : "memory");
-}
 // 16-byte global store issued from inline asm: the compiler's wait-count tracking does not see
 // it, so pending output stores never turn its waits for tile loads into full drains (loads and
 // stores share the counter, and with both pending it would wait for zero). Every wait the
@@ -169,10 +152,6 @@ __device__ __forceinline__ void dma_b128(uint32_t voff, __amdgpu_buffer_rsrc_t r
 __device__ __forceinline__ void gstore_b128(void* p, u32x4 v) {
     asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" :: "v"(p), "v"(v) : "memory");
 }
-__device__ __forceinline__ uint32_t lds_byte_addr(const void* p) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-
 __device__ __forceinline__ int sigma16(int t) {  // swap bits 2 and 3 (token order in V^T rows)
     return (t & ~12) | ((t & 4) << 1) | ((t & 8) >> 1);
 }
@@ -1773,8 +1752,8 @@ static int varlen_prefill_impl(void* out, int out_dtype, int64_t o_stride_tok,
         return launch_prefill_f32_mfma(out_dtype, out, o_stride_tok, o_stride_head, q, q_stride_tok,
                                        q_stride_head, k_pool, v_pool, cu_seqlens_q, nullptr,
                                        kv_lens, block_tables, max_blocks_per_seq, num_seqs,
-                                       max_seqlen_q, num_heads, n_rep, head_dim, block_size,
-                                       num_slots, scale, s);
+                                       max_seqlen_q, total_q, num_heads, n_rep, head_dim,
+                                       block_size, num_slots, scale, s);
     if (!mfma && q_rows) {
         set_error("varlen_prefill: row indices need the matrix-core path");
         return FLOUR_ERR_UNSUPPORTED;

@@ -56,6 +56,40 @@ def test_prefill_f32_matrix_cores_match_oracle(device, H, G, D, bs, lens, prefix
     assert max_abs <= 1e-5
 
 
+@pytest.mark.parametrize("H,G,D,bs,lens,prefix,short", [
+    (128, 128, 64, 16, [129, 1, 127, 260], 0, None),         # n_rep 1: 128-row items, their edges
+    (128, 64, 128, 32, [64, 65, 1, 63, 200, 130], 32, 3),    # n_rep 2: 64-row items, 32-token pages
+    (128, 32, 128, 16, [32, 33, 31, 1, 97, 330], 16, None),  # n_rep 4: 32-row items
+    (112, 16, 64, 48, [300, 230, 2], 48, 1),                 # n_rep 7: a wave without a head
+    (96, 32, 128, 16, [680, 100], 0, None),                  # n_rep 3: one head an item
+    (64, 16, 64, 16, [17] * 64, 128, 40),                    # 64 sequences
+])
+def test_prefill_f32_tiles_match_oracle(device, H, G, D, bs, lens, prefix, short):
+    """Batches of two items per CU or more (the tile kernel): against the oracle, with rows past
+    each sequence's positions holding garbage, a sequence whose kv length is below its query count,
+    a bad block id past the used pages and 16-bit outputs."""
+    c = make_prefill(len(lens), H, G, D, bs, (1, 1), prefix=prefix, dtype=torch.float32,
+                     seed=H + D + bs, device="cuda:0", q_lens=lens)  # (every pool row is filled)
+    used = torch.zeros(c.k_pool.shape[1], dtype=torch.bool)
+    for s, n in enumerate(c.kv_lens.tolist()):
+        j = torch.arange(n)
+        used[c.block_tables[s].cpu()[j // bs].long() * bs + j % bs] = True
+        c.block_tables[s, (n + bs - 1) // bs:] = -7
+    c.k_pool[:, ~used.to(device)] = float("nan")
+    c.v_pool[:, ~used.to(device)] = float("inf")
+    if short is not None:
+        c.kv_lens[short] = lens[short] - 1
+    got = _run(c)
+    max_abs, _ = errors(to_np(got), _oracle(c))
+    print(f"fp32 tiles H={H} G={G} D={D}: max_abs={max_abs:.3e}", flush=True)
+    assert max_abs <= 1e-5
+    if short is not None:
+        a, b = c.cu_seqlens_q[short:short + 2].tolist()
+        assert not got[a:b].any()
+    for dt in (torch.bfloat16, torch.float16):
+        assert torch.equal(_run(c, dt), got.to(dt))
+
+
 def test_prefill_f32_matches_the_vector_kernel(device):
     """The matrix-core and vector fp32 paths agree to the fp32 bound on the same batch."""
     c = _case(8, 2, 128, 16, [200, 31, 64], 16, seed=3)
