@@ -29,6 +29,7 @@
 #include <math.h>
 
 #include "flour_common.h"
+#include "prefill_items.h"
 
 namespace flour {
 
@@ -41,29 +42,6 @@ __host__ __device__ constexpr int f32m_waves(int d) { return d == 64 ? 8 : 4; }
 
 __device__ __forceinline__ f32x16 mfma32x32x2_f32(float a, float b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-// Stores N consecutive outputs (N = 2 or 4) from fp32.
-template <int N>
-__device__ __forceinline__ void store_run(void* out, int out_dtype, int64_t idx, const float* v) {
-    if (out_dtype == FLOUR_DTYPE_F32) {
-        if constexpr (N == 4)
-            *reinterpret_cast<f32x4*>(static_cast<float*>(out) + idx) = f32x4{v[0], v[1], v[2], v[3]};
-        else
-            *reinterpret_cast<f32x2*>(static_cast<float*>(out) + idx) = f32x2{v[0], v[1]};
-    } else if (out_dtype == FLOUR_DTYPE_BF16) {
-        if constexpr (N == 4)
-            *reinterpret_cast<u32x2*>(static_cast<bf16_t*>(out) + idx) =
-                u32x2{pack2<bf16_t>(v[0], v[1]), pack2<bf16_t>(v[2], v[3])};
-        else
-            *reinterpret_cast<uint32_t*>(static_cast<bf16_t*>(out) + idx) = pack2<bf16_t>(v[0], v[1]);
-    } else {
-        if constexpr (N == 4)
-            *reinterpret_cast<u32x2*>(static_cast<f16_t*>(out) + idx) =
-                u32x2{pack2<f16_t>(v[0], v[1]), pack2<f16_t>(v[2], v[3])};
-        else
-            *reinterpret_cast<uint32_t*>(static_cast<f16_t*>(out) + idx) = pack2<f16_t>(v[0], v[1]);
-    }
 }
 
 template <int D>
@@ -294,34 +272,17 @@ __global__ __launch_bounds__(F32T_WAVES * 64, 2) void prefill_f32_tile_kernel(
     const uint32_t head_bytes = (uint32_t)num_slots * D * 4u;
     const int G = gridDim.x;
 
-    // The items, longest first: tile index (level) by decreasing level, then sequence, then head
-    // group. Every wave walks the levels by itself with one sequence per lane.
-    const int my_c0 = cu_seqlens_q[min(lane, num_seqs)];
-    const int my_rows = lane < num_seqs ? cu_seqlens_q[lane + 1] - my_c0 : 0;
-    const int my_kv = lane < num_seqs ? min(kv_lens[lane], max_blocks * block_size) : 0;
-    const int my_tiles = my_rows > 0 ? (my_rows + rows - 1) / rows : 0;
-    int level = n_qt - 1, base = 0;  // items of the levels above `level`
-    uint64_t there = __ballot(my_tiles > level);
+    ItemWalk items;
+    items.start(cu_seqlens_q, kv_lens, num_seqs, max_blocks * block_size, rows, n_qt, per_row, lane);
     if (ks == 0) __builtin_amdgcn_s_setprio(1);
 
     for (int round = 0;; round++) {
-        // a snake over the list: even rounds in workgroup order, odd ones reversed
-        const int idx = round * G + ((round & 1) ? G - 1 - (int)blockIdx.x : (int)blockIdx.x);
-        while (level >= 0 && idx >= base + per_row * __popcll(there)) {
-            base += per_row * __popcll(there);
-            level--;
-            there = __ballot(my_tiles > level);
-        }
-        if (level < 0) break;  // past the list, and so is every later round's index
-        const int rank = (idx - base) / per_row, x = idx - base - rank * per_row;
-        const uint64_t nth =
-            __ballot(((there >> lane) & 1) && __popcll(there & ((1ull << lane) - 1)) == rank);
-        const int s = __ffsll((unsigned long long)nth) - 1;
-        const int qt = level;
+        int s, qt, x;
+        if (!items.find(ItemWalk::deal(round, G, blockIdx.x), lane, s, qt, x)) break;
         const int kvh = x / groups, h0 = (x - kvh * groups) * hw;
-        const int c0 = __builtin_amdgcn_readlane(my_c0, s);
-        const int q_len = __builtin_amdgcn_readlane(my_rows, s);
-        const int kv_len = __builtin_amdgcn_readlane(my_kv, s);
+        const int c0 = __builtin_amdgcn_readlane(items.c0, s);
+        const int q_len = __builtin_amdgcn_readlane(items.rows, s);
+        const int kv_len = __builtin_amdgcn_readlane(items.kv, s);
         const int off = kv_len - q_len;  // row i sees positions j <= off + i
         const bool reads = kv_len >= q_len;
         const int kv_end = reads ? off + min(qt * rows + rows, q_len) : 0;  // the item's range
@@ -510,13 +471,6 @@ __global__ __launch_bounds__(F32T_WAVES * 64, 2) void prefill_f32_tile_kernel(
     }
 }
 
-// Query heads per item of the tile kernel: 4 or 2 where at most one wave in eight is left without
-// a head, else 1.
-static int f32_tile_heads(int n_rep) {
-    if (n_rep % 4 == 0 || (n_rep % 4 == 3 && n_rep > 3)) return 4;
-    return n_rep % 2 == 0 ? 2 : 1;
-}
-
 static int device_cus_f32() {
     static int cached[64] = {0};
     int dev = 0;
@@ -560,7 +514,7 @@ int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh
     // 157, 2 x 1,024 203 / 168; 8 / 8 of 64, 1 x 1,024 (1/4) 29 / 77, 8 x 1,024 (2) 123 / 102; 16 /
     // 16 of 128, 4 x U[512, 1,024] (1.5) 130 / 136; 14 / 2 of 64, 8 x U[256, 1,024] (2.5) 113 / 114.
     // Its item list holds up to 64 sequences, its loads 32-bit offsets.
-    const int hw = f32_tile_heads(n_rep), kv_heads = num_heads / n_rep;
+    const int hw = item_heads(n_rep), kv_heads = num_heads / n_rep;
     const int rows = F32M_QT * (4 / hw);
     const int64_t per_row = (int64_t)kv_heads * ((n_rep + hw - 1) / hw);
     const int64_t cus = device_cus_f32();

@@ -253,6 +253,29 @@ __device__ __forceinline__ float sum_across_halves(float x) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// Stores N consecutive outputs (N = 2 or 4) from fp32.
+template <int N>
+__device__ __forceinline__ void store_run(void* out, int out_dtype, int64_t idx, const float* v) {
+    if (out_dtype == FLOUR_DTYPE_F32) {
+        if constexpr (N == 4)
+            *reinterpret_cast<f32x4*>(static_cast<float*>(out) + idx) = f32x4{v[0], v[1], v[2], v[3]};
+        else
+            *reinterpret_cast<f32x2*>(static_cast<float*>(out) + idx) = f32x2{v[0], v[1]};
+    } else if (out_dtype == FLOUR_DTYPE_BF16) {
+        if constexpr (N == 4)
+            *reinterpret_cast<u32x2*>(static_cast<bf16_t*>(out) + idx) =
+                u32x2{pack2<bf16_t>(v[0], v[1]), pack2<bf16_t>(v[2], v[3])};
+        else
+            *reinterpret_cast<uint32_t*>(static_cast<bf16_t*>(out) + idx) = pack2<bf16_t>(v[0], v[1]);
+    } else {
+        if constexpr (N == 4)
+            *reinterpret_cast<u32x2*>(static_cast<f16_t*>(out) + idx) =
+                u32x2{pack2<f16_t>(v[0], v[1]), pack2<f16_t>(v[2], v[3])};
+        else
+            *reinterpret_cast<uint32_t*>(static_cast<f16_t*>(out) + idx) = pack2<f16_t>(v[0], v[1]);
+    }
+}
+
 // ------------------------------------------------------------------ host-side error state
 // Both are noexcept: the message lives in a fixed per-thread buffer.
 void set_error(const char* fmt, ...) noexcept __attribute__((format(printf, 1, 2)));

@@ -153,3 +153,39 @@ def test_prefill_d64_reference_layout(device):
     ref, rows = oracle_prefill(c)
     max_abs, rel = errors(to_np(out)[rows], ref)
     assert max_abs <= 2e-3 and rel <= 1e-3
+
+
+@pytest.mark.parametrize("H,G,bs,lens,prefix,short", [
+    (14, 2, 16, [1000], 0, None),                     # one prompt, two slots an item (GQA 7)
+    (14, 2, 16, [511, 130, 64, 33, 1, 385, 500, 480], 0, 3),  # four slots, row and step edges
+    (8, 8, 32, [129, 128, 1, 65], 32, None),          # one head an item, 32-token pages
+    (6, 2, 48, [200, 31], 96, 1),                     # n_rep 3, 48-token pages
+    (16, 1, 16, [40] * 64, 256, 7),                   # n_rep 16, 64 sequences
+    (12, 2, 16, [300], 1008, None),                   # n_rep 6, a prefix that ends inside a step
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_small_batches(device, dtype, H, G, bs, lens, prefix, short):
+    """Batches small enough for the 32-row items: against the oracle, with garbage in every row past
+    the sequences' positions, bad block ids past the used pages, a sequence whose kv length is below
+    its query count, and both schedules alike."""
+    c = make_prefill(len(lens), H, G, D, bs, (1, 1), prefix=prefix, dtype=dtype, seed=H + bs,
+                     device=device, q_lens=lens)  # (every pool row is filled)
+    used = torch.zeros(c.k_pool.shape[1], dtype=torch.bool)
+    for s, n in enumerate(c.kv_lens.tolist()):
+        j = torch.arange(n)
+        used[c.block_tables[s].cpu()[j // bs].long() * bs + j % bs] = True
+        c.block_tables[s, (n + bs - 1) // bs:] = -7
+    c.k_pool[:, ~used.to(device)] = float("nan")
+    c.v_pool[:, ~used.to(device)] = float("inf")
+    if short is not None:
+        c.kv_lens[short] = lens[short] - 1
+    got = go(c)
+    ref, rows = oracle_prefill(c, None)
+    max_abs, rel = errors(to_np(got)[rows], ref)
+    print(f"small batch H={H} G={G} {dtype}: max_abs={max_abs:.3e} rel_l2={rel:.3e}", flush=True)
+    assert max_abs <= 2e-3 and rel <= 1e-3
+    if short is not None:
+        a, b = c.cu_seqlens_q[short:short + 2].tolist()
+        assert not got[a:b].any()
+    assert torch.equal(got, go(c, persistent=0))
+    assert torch.equal(go(c, out_dtype=dtype), got.to(dtype))
