@@ -1194,10 +1194,11 @@ static int paged_decode_impl(void* out, int out_dtype, const void* q, const void
     const bool ws_ok = ws_from_scratch ? need <= DEC_SCRATCH_BYTES
                                        : workspace && workspace_bytes >= need &&
                                              ((uintptr_t)workspace % 256) == 0;
+    // (an fp32 call without a workspace never touches the library's shared one)
     const bool f32_split =
-        dtype == FLOUR_DTYPE_F32 && decode_f32_split(head_dim, block_size, n_rep, batch, num_heads,
-                                                     num_slots, max_context_len, q, k_pool, v_pool,
-                                                     ws_ok);
+        dtype == FLOUR_DTYPE_F32 &&
+        decode_f32_split(head_dim, block_size, n_rep, batch, num_heads, num_slots, max_context_len,
+                         q, k_pool, v_pool, ws_ok && !ws_from_scratch);
     if (!mfma && !f32_split) {
         // one query row per sequence: cu_seqlens == nullptr
         const int64_t qs = (int64_t)num_heads * head_dim;

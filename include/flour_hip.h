@@ -150,7 +150,8 @@ int flour_hip_paged_decode(void* out, int out_dtype, const void* q, const void* 
  * until the process ends). Arguments, results and kernels are those of flour_hip_paged_decode.
  * A call whose workspace would exceed that size fails with FLOUR_ERR_WORKSPACE before any
  * launch (at 256 CUs every shape the MFMA path takes fits; larger GQA groups or batches than
- * that would need flour_hip_paged_decode). Every call on one GPU shares that GPU's array:
+ * that would need flour_hip_paged_decode). fp32 pools run on the vector kernel here, whatever
+ * the length. Every call on one GPU shares that GPU's array:
  * calls that overlap in time on one GPU (different streams, or threads without ordering) race
  * and give wrong results. Nothing needs to start at zero; the array keeps the last call's
  * contents.

@@ -110,6 +110,25 @@ def test_decode_fp32_split(device, H, G, D, bs, ctx):
         assert torch.equal(run(c, dt), got.to(dt))
 
 
+def test_decode_fp32_split_on_two_streams(device):
+    """fp32 steps without a workspace argument share none: overlapping calls on two streams give
+    what each gives alone."""
+    cases = [make_decode(4, 32, 8, 128, 16, (1000, 4000), dtype=torch.float32, seed=s, device=device)
+             for s in (1, 2)]
+    alone = [run(c) for c in cases]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    outs = [[], []]
+    for _ in range(8):
+        for i, c in enumerate(cases):
+            with torch.cuda.stream(streams[i]):
+                outs[i].append(ops.paged_decode(c.q, c.k_pool, c.v_pool, c.block_tables,
+                                                c.context_lens, c.scale, c.max_context_len))
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(o, alone[i]) for o in outs[i])
+
+
 @pytest.mark.parametrize("ctx", [[1], [33], [65, 2], [100], [1000], [5000], [40] * 65])
 def test_decode_few_chunks(device, ctx):
     """Chunk lists shorter than the grid (at least two chunks a range) and merges split over
