@@ -8,6 +8,8 @@
 // sees kv position j iff j <= kv_len - q_len + i (cpu.rs:68, :88-95); query head h reads kv
 // head h / n_rep (repeat_kv, cpu.rs:5-13).
 //
+// Small batches at head_dim 64 run in prefill_thin.hip, fp32 pools in attn_f32_mfma.hip.
+//
 // Design (head_dim 128, block_size a multiple of 16):
 //  * One workgroup (8 waves) per (128-row query tile, pair of query heads that share a kv
 //    head, sequence); wave w owns 32 query rows of head w / 4, and every K/V tile staged in
