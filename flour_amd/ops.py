@@ -207,7 +207,9 @@ def prepare_paged_decode(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Te
                          block_size: int = 16):
     """Validates the arguments of paged_decode once and returns a callable that relaunches the
     same decode step (same tensors, current stream at preparation time) with no per-call
-    Python work beyond the C call, as a serving loop that reuses its buffers would."""
+    Python work beyond the C call, as a serving loop that reuses its buffers would. The callable
+    keeps the workspace's present buffer alive, also when the workspace grows or goes; the
+    caller keeps the tensors."""
     _need_cuda(q, k_pool, v_pool, block_tables, context_lens, out)
     _need_i32(block_tables, context_lens)
     B, H, D = q.shape
@@ -229,6 +231,7 @@ def prepare_paged_decode(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Te
         if rc:
             check(rc)
 
+    run.workspace = ws  # the buffer whose address args holds
     return run
 
 
