@@ -197,6 +197,20 @@ __device__ __forceinline__ int64_t range_count(int64_t total, int64_t cap) {
     return half < 1 ? 1 : (half < cap ? half : cap);
 }
 
+// Running maxima start at the lowest finite value: with scores of -inf alone (K rows that hold -inf,
+// products that overflow) the maximum stays finite, every weight is exp2(-inf) = 0 and no
+// difference of infinities reaches the sums. It costs nothing where a select per chunk would.
+static constexpr float DEC_M0 = -3.402823466e38f;
+
+// What a row is divided by: its sum of weights, or 1 where that is 0 (no score above -inf: a zero
+// row). Over fp32 pools an undefined sum (scores of NaN or +inf) gives a zero row too, as on the
+// vector kernel (attn_simt.hip): the caller clears the row wherever !(sum > 0). The 16-bit pools
+// hand a NaN on.
+template <bool F32>
+__device__ __forceinline__ float divisor(float sum) {
+    return (F32 ? !(sum > 0.0f) : sum == 0.0f) ? 1.0f : sum;
+}
+
 __device__ __forceinline__ f32x4 mfma16x16x4_f32(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
@@ -404,7 +418,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
                                   : u32x4{0, 0, 0, 0};
     };
 
-    float m = -INFINITY, lsum = 0.0f;
+    float m = DEC_M0, lsum = 0.0f;
     f32x4 acc[NV];
 #pragma unroll
     for (int nn = 0; nn < NV; nn++) acc[nn] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -556,7 +570,10 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
                 const int64_t row = ws.rows ? (int64_t)ws.rows[b] : (int64_t)b;
                 TO* o = out + (row * num_heads + (int64_t)g * n_rep + lc) * D +
                         (F32 ? 16 : D / 4) * lgo;
-                const float inv = 1.0f / lsum;
+                const float inv = 1.0f / divisor<F32>(lsum);
+                if (F32 && !(lsum > 0.0f))
+#pragma unroll
+                    for (int nn = 0; nn < NV; nn++) acc[nn] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     if constexpr (F32) {
@@ -602,7 +619,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
                 }
             }
         }
-        m = -INFINITY;
+        m = DEC_M0;
         lsum = 0.0f;
 #pragma unroll
         for (int nn = 0; nn < NV; nn++) acc[nn] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -791,7 +808,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_mfma_kernel(
 // workgroup's waves split them, since one wave reads them 8 rows a memory round trip, and fold
 // their states through LDS; with one wave there is no LDS and no barrier.
 static constexpr int DEC_MERGE_WAVES = 8;
-template <typename TO, int D>
+template <typename TO, int D, bool F32>
 __global__ __launch_bounds__(64 * DEC_MERGE_WAVES) void paged_decode_merge_kernel(
     TO* __restrict__ out, int batch, int num_heads, int kv_heads, int n_rep, int nwg_i,
     DecodeWs ws) {
@@ -825,7 +842,7 @@ __global__ __launch_bounds__(64 * DEC_MERGE_WAVES) void paged_decode_merge_kerne
     if (f == l) return;  // finished inside one wave range
     const int np = (int)(l - f + 1);  // ranges f..l, none of them empty
 
-    float M = -INFINITY, L = 0.0f, O[E];
+    float M = DEC_M0, L = 0.0f, O[E];
 #pragma unroll
     for (int i = 0; i < E; i++) O[i] = 0.0f;
     const int fslot = (int)(f_first ? 2 * f : 2 * f + 1);  // the first piece always exists
@@ -867,7 +884,7 @@ __global__ __launch_bounds__(64 * DEC_MERGE_WAVES) void paged_decode_merge_kerne
         const float m_new = fmaxf(M, wave_max(mx));
         const float w = (slot >= 0) ? fast_exp2(mx - m_new) : 0.0f;
         const float bl = wave_sum(w * lx);
-        const float c_old = (M == -INFINITY) ? 0.0f : fast_exp2(M - m_new);
+        const float c_old = fast_exp2(M - m_new);
         L = L * c_old + bl;
 #pragma unroll
         for (int i = 0; i < E; i++) O[i] *= c_old;
@@ -896,7 +913,7 @@ __global__ __launch_bounds__(64 * DEC_MERGE_WAVES) void paged_decode_merge_kerne
         }
         M = m_new;
     }
-    if (waves > 1) {  // the waves' states, folded by the first (a wave without pieces has M = -inf)
+    if (waves > 1) {  // the waves' states, folded by the first (it always has pieces)
         __shared__ float wM[DEC_MERGE_WAVES], wL[DEC_MERGE_WAVES];
         __shared__ float wO[DEC_MERGE_WAVES][E][64];
         if (lane == 0) {
@@ -936,7 +953,10 @@ __global__ __launch_bounds__(64 * DEC_MERGE_WAVES) void paged_decode_merge_kerne
         }
     }
 #pragma unroll
-    for (int i = 0; i < E; i++) o[i] = from_f32<TO>(O[i] / L);
+    for (int i = 0; i < E; i++) {
+        const float x = O[i] / divisor<F32>(L);
+        o[i] = from_f32<TO>(F32 && !(L > 0.0f) ? 0.0f : x);
+    }
 }
 
 // Waves per merge workgroup: about eight pieces (one memory round trip) each, for twice the mean
@@ -975,8 +995,9 @@ static int launch_decode_mfma_d(void* out, const void* q, const void* k_pool, co
     int rc = check_hip(hipGetLastError(), "paged_decode launch");
     if (rc != FLOUR_OK) return rc;
     const int mw = decode_merge_waves(grid, batch, kv_heads);
-    paged_decode_merge_kernel<TO, D><<<dim3(num_heads, batch), dim3(64 * mw), 0, stream>>>(
-        static_cast<TO*>(out), batch, num_heads, kv_heads, n_rep, grid, ws);
+    paged_decode_merge_kernel<TO, D, std::is_same<T, float>::value>
+        <<<dim3(num_heads, batch), dim3(64 * mw), 0, stream>>>(
+            static_cast<TO*>(out), batch, num_heads, kv_heads, n_rep, grid, ws);
     return check_hip(hipGetLastError(), "paged_decode merge launch");
 }
 

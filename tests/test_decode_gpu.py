@@ -129,6 +129,54 @@ def test_decode_fp32_split_on_two_streams(device):
         assert all(torch.equal(o, alone[i]) for o in outs[i])
 
 
+def _scores_of(c, rows, value):
+    """Puts ``value`` into dim 0 of the K rows of (sequence, position) pairs ``rows`` and makes
+    dim 0 of every query positive, so that those positions' scores are +-inf or NaN."""
+    c.q[..., 0] = c.q[..., 0].abs() + 0.1
+    for s, j in rows:
+        c.k_pool[:, int(c.block_tables[s, j // c.block_size]) * c.block_size + j % c.block_size, 0] = value
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,D,lead", [
+    (32, 8, 128, [(2100, 16), (2100, 33), (1500, 1500), (40, 40), (700, 0), (900, 600)]),
+    (14, 2, 64, [(4000, 2100)]),   # one sequence: whole pieces, and whole shares of the merge
+    (8, 8, 64, [(2500, 40), (2500, 2500), (3, 2)]),
+    (8, 2, 128, [(700, 32)] + [(5, 0)] * 70),  # more than 64 sequences
+])
+def test_decode_scores_of_minus_infinity(device, dt, H, G, D, lead):
+    """Scores of -inf over a context's first positions (a chunk, a piece, all of it) weigh nothing,
+    and a context without any other score gives a zero row, as in the oracle."""
+    ctx = [n for n, _ in lead]
+    c = make_decode(len(ctx), H, G, D, 16, (1, 1), dtype=dt, seed=H + D, device=device,
+                    context_lens=ctx)
+    _scores_of(c, [(s, j) for s, (_, k) in enumerate(lead) for j in range(k)], float("-inf"))
+    ref = oracle_decode(c)
+    assert np.isfinite(ref).all()
+    got = to_np(run(c, torch.float32))
+    assert np.isfinite(got).all()
+    max_abs, rel = errors(got, ref)
+    print(f"-inf scores {dt} H={H} G={G} D={D}: max_abs={max_abs:.3e} rel={rel:.3e}", flush=True)
+    assert max_abs <= (1e-5 if dt == torch.float32 else 2e-3) and rel <= 1e-3
+    for s, (n, k) in enumerate(lead):
+        if n == k:
+            assert not got[s].any()
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("ctx", [[2500], [1200, 40, 2500]])
+def test_decode_fp32_undefined_scores(device, ctx, value):
+    """An fp32 context with a score of NaN or +inf has no softmax: a zero row, as the oracle's
+    guard (a sum that is not positive) and the vector kernel give."""
+    c = make_decode(len(ctx), 32, 8, 128, 16, (1, 1), dtype=torch.float32, seed=17, device=device,
+                    context_lens=ctx)
+    _scores_of(c, [(0, 700)], value)
+    ref = oracle_decode(c)
+    got = to_np(run(c))
+    assert not ref[0].any() and not got[0].any()
+    assert errors(got, ref)[0] <= 1e-5
+
+
 @pytest.mark.parametrize("ctx", [[1], [33], [65, 2], [100], [1000], [5000], [40] * 65])
 def test_decode_few_chunks(device, ctx):
     """Chunk lists shorter than the grid (at least two chunks a range) and merges split over
