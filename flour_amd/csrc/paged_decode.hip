@@ -1157,13 +1157,13 @@ bool decode_mfma_supported(int dtype, int head_dim, int block_size, int n_rep, i
 // than on the vector kernel, which needs no workspace but gives each (sequence, kv head) one
 // workgroup.
 static bool decode_f32_split(int head_dim, int block_size, int n_rep, int batch, int num_heads,
-                             int64_t num_slots, int max_context_len, const void* q,
-                             const void* k_pool, const void* v_pool, bool ws_ok) {
+                             int64_t num_slots, int max_context_len, const void* out,
+                             const void* q, const void* k_pool, const void* v_pool, bool ws_ok) {
     if (!ws_ok || (head_dim != 128 && head_dim != 64) || block_size % 16 != 0 || n_rep > 16 ||
         batch > DEC_MAX_BATCH || num_heads > 65535 ||
         num_slots * head_dim * 4 > (int64_t)0x7fffffff ||
-        (((uintptr_t)q | (uintptr_t)k_pool | (uintptr_t)v_pool) & 15) != 0)
-        return false;
+        (((uintptr_t)out | (uintptr_t)q | (uintptr_t)k_pool | (uintptr_t)v_pool) & 15) != 0)
+        return false;  // (its output stores are up to 16 bytes wide, the vector kernel's one element)
     // The vector kernel's time goes with a workgroup's kv length x queries (n_rep, as a power of
     // two) x head_dim; a split step takes ~9 us and its bytes. Vector / split in us: 1 x 256 tokens of
     // 32 / 8 heads of 128 14.5 / 10.3 (64 tokens: 7.4 / 9.8), 14 / 2 heads of 64 13.4 / 8.8 (64: 8.3 /
@@ -1219,7 +1219,7 @@ static int paged_decode_impl(void* out, int out_dtype, const void* q, const void
     const bool f32_split =
         dtype == FLOUR_DTYPE_F32 &&
         decode_f32_split(head_dim, block_size, n_rep, batch, num_heads, num_slots, max_context_len,
-                         q, k_pool, v_pool, ws_ok && !ws_from_scratch);
+                         out, q, k_pool, v_pool, ws_ok && !ws_from_scratch);
     if (!mfma && !f32_split) {
         // one query row per sequence: cu_seqlens == nullptr
         const int64_t qs = (int64_t)num_heads * head_dim;

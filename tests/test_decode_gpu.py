@@ -177,6 +177,25 @@ def test_decode_fp32_undefined_scores(device, ctx, value):
     assert errors(got, ref)[0] <= 1e-5
 
 
+def test_decode_fp32_unaligned_output(device):
+    """An fp32 step whose output is not 16-byte aligned is taken as before and gives the vector
+    kernel's result."""
+    from flour_amd import _lib
+    c = make_decode(3, 32, 8, 128, 16, (1, 1), dtype=torch.float32, seed=18, device=device,
+                    context_lens=[1000, 5, 300])
+    p, n = ops._ptr, c.q.numel()
+    outs = [torch.full((n + 1,), 7.0, device=device) for _ in range(2)]
+    ws = ops.DecodeWorkspace(device).get(ops.decode_workspace_bytes(3, 32, 8, 128, 1000))
+    for buf, w in zip(outs, (ws, None)):
+        _lib.check(_lib.lib().flour_hip_paged_decode(
+            buf.data_ptr() + 4, 0, p(c.q), p(c.k_pool), p(c.v_pool), p(c.block_tables),
+            c.block_tables.shape[1], p(c.context_lens), 3, 32, 8, 128, 16, c.k_pool.shape[1], 1000,
+            c.scale, 0, None if w is None else p(w), 0 if w is None else w.numel(), ops._stream()))
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]) and float(outs[0][0]) == 7.0
+    assert errors(to_np(outs[0][1:].view_as(c.q)), oracle_decode(c))[0] <= 1e-5
+
+
 @pytest.mark.parametrize("ctx", [[1], [33], [65, 2], [100], [1000], [5000], [40] * 65])
 def test_decode_few_chunks(device, ctx):
     """Chunk lists shorter than the grid (at least two chunks a range) and merges split over
