@@ -184,20 +184,22 @@ def paged_decode(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
     out_dtype = out_dtype or q.dtype
     if out is None:
         out = torch.empty((B, H, D), dtype=out_dtype, device=q.device)
-    nbytes = decode_workspace_bytes(B, H, G, D, max_context_len)
-    if workspace is None and q.dtype == torch.float32 and max_context_len * D >= 16384:
-        # a step that may be split: scratch of its own, in the current stream's order (short fp32
-        # steps read none, and none has to share the default workspace between streams)
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+    if workspace is None and q.dtype == torch.float32:
+        # Scratch of its own, in the current stream's order: fp32 steps without a workspace
+        # argument share nothing between streams. Steps that the library never splits (shorter
+        # than this, other heads) pass none, and run on the vector kernel.
+        may_split = max_context_len * D >= 16384 and D in (64, 128) and H <= 16 * G
+        ws = torch.empty(decode_workspace_bytes(B, H, G, D, max_context_len), dtype=torch.uint8,
+                         device=q.device) if may_split else None
     else:
         if workspace is None:
             workspace = _default_ws.setdefault(q.device.index or 0, DecodeWorkspace(q.device))
-        ws = workspace.get(nbytes)
+        ws = workspace.get(decode_workspace_bytes(B, H, G, D, max_context_len))
     check(lib().flour_hip_paged_decode(_ptr(out), dtype_code(out.dtype), _ptr(q), _ptr(k_pool),
                                        _ptr(v_pool), _ptr(block_tables), block_tables.shape[1],
                                        _ptr(context_lens), B, H, G, D, block_size, num_slots,
                                        max_context_len, float(scale), dtype_code(q.dtype),
-                                       _ptr(ws), ws.numel(), _stream()))
+                                       _ptr(ws), 0 if ws is None else ws.numel(), _stream()))
     return out
 
 

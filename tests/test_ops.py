@@ -65,3 +65,26 @@ def test_prepared_decode_owns_its_workspace(recorded, dtype, then):
     del step
     gc.collect()
     assert buf() is None
+
+
+@pytest.mark.parametrize("max_ctx", [1, 128, 255, 256, 257, 4096])
+def test_fp32_decode_without_a_workspace_shares_none(recorded, max_ctx):
+    """Two fp32 steps without a workspace argument never get the same scratch, whatever rule the
+    library has for the length from which it uses one: their own, or none."""
+    args = decode_args(torch.float32, max_ctx)
+    held = []
+    for _ in range(2):
+        ops.paged_decode(*args)
+        *_, address, nbytes, _ = recorded.calls[-1]
+        held.append((address.value or 0, nbytes))
+    assert not ops._default_ws
+    for address, nbytes in held:
+        assert (address == 0) == (nbytes == 0)
+
+
+def test_16_bit_decode_without_a_workspace_reuses_the_default(recorded):
+    args = decode_args(torch.bfloat16, 300)
+    for _ in range(2):
+        ops.paged_decode(*args)
+    a, b = (call[-3].value for call in recorded.calls)
+    assert a == b == ops._default_ws[0].buf.data_ptr()
