@@ -976,13 +976,13 @@ static int launch_decode_mfma_d(void* out, const void* q, const void* k_pool, co
                                 hipStream_t stream) {
     const size_t lds = (size_t)(batch + 1) * sizeof(int);
     const bool fuse = ws.k_new != nullptr;
-    if (fuse && block_size != 16) {  // paged_decode_write_kv takes 16-token pages only
-        set_error("paged_decode: the fused KV write needs 16-token pages");
+    if (fuse && (block_size != 16 || std::is_same<T, float>::value)) {
+        set_error("paged_decode: the fused KV write needs 16-token pages of a 16-bit pool");
         return FLOUR_ERR_UNSUPPORTED;
     }
     auto kern = block_size == 16 ? paged_decode_mfma_kernel<T, TO, true, D, false>
                                  : paged_decode_mfma_kernel<T, TO, false, D, false>;
-    if constexpr (!std::is_same<T, float>::value)  // (fp32 pools take no fused write)
+    if constexpr (!std::is_same<T, float>::value)
         if (fuse) kern = paged_decode_mfma_kernel<T, TO, true, D, true>;
     // no more waves than ranges (range_count) for contexts of max_ctx
     const int64_t chunk = dec_chunk(sizeof(T));
