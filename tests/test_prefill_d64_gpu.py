@@ -189,3 +189,13 @@ def test_small_batches(device, dtype, H, G, bs, lens, prefix, short):
         assert not got[a:b].any()
     assert torch.equal(got, go(c, persistent=0))
     assert torch.equal(go(c, out_dtype=dtype), got.to(dtype))
+
+
+@pytest.mark.parametrize("bound", [1000, 1024, 40000, 65536])
+def test_small_batch_with_a_loose_row_bound(device, bound):
+    """max_seqlen_q is a bound: one far above the longest sequence changes nothing."""
+    c = make_prefill(3, 14, 2, D, 16, (1, 1), prefix=32, dtype=torch.bfloat16, seed=97,
+                     device=device, q_lens=[400, 64, 9])
+    tight = go(c)
+    c.max_seqlen_q = bound
+    assert torch.equal(go(c), tight)

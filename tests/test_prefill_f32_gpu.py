@@ -90,6 +90,16 @@ def test_prefill_f32_tiles_match_oracle(device, H, G, D, bs, lens, prefix, short
         assert torch.equal(_run(c, dt), got.to(dt))
 
 
+@pytest.mark.parametrize("bound", [700, 20000, 1 << 20])
+def test_prefill_f32_tiles_with_a_loose_row_bound(device, bound):
+    """max_seqlen_q is a bound: one far above the longest sequence changes nothing."""
+    c = make_prefill(4, 64, 16, 128, 16, (1, 1), prefix=0, dtype=torch.float32, seed=98,
+                     device="cuda:0", q_lens=[680, 600, 1, 300])
+    tight = _run(c)
+    c.max_seqlen_q = bound
+    assert torch.equal(_run(c), tight)
+
+
 def test_prefill_f32_matches_the_vector_kernel(device):
     """The matrix-core and vector fp32 paths agree to the fp32 bound on the same batch."""
     c = _case(8, 2, 128, 16, [200, 31, 64], 16, seed=3)
