@@ -485,7 +485,9 @@ static int device_cus_f32() {
     return cached[dev];
 }
 
-static int g_prefill_f32_mfma = 1;  // a test / tuning switch
+// 0: the vector kernel, 1: by the rules below, 2 / 3: never / always (within its limits) the tile
+// kernel. A test / tuning switch.
+static int g_prefill_f32_mfma = 1;
 
 bool prefill_f32_mfma_supported(int dtype, int head_dim, int num_seqs, int max_seqlen_q,
                                 int block_size, int64_t num_slots) {
@@ -518,9 +520,10 @@ int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh
     const int rows = F32M_QT * (4 / hw);
     const int64_t per_row = (int64_t)kv_heads * ((n_rep + hw - 1) / hw);
     const int64_t cus = device_cus_f32();
-    const bool tiled = !q_rows && num_seqs <= 64 && num_slots * head_dim * 4 <= 0x7fffffff &&
-                       per_row * (total_q / rows) >= 2 * cus &&
-                       per_row * num_seqs * ((int64_t)max_seqlen_q / rows + 1) <= 0x3fffffff;
+    const bool fits = !q_rows && num_seqs <= 64 && num_slots * head_dim * 4 <= 0x7fffffff &&
+                      per_row * num_seqs * ((int64_t)max_seqlen_q / rows + 1) <= 0x3fffffff;
+    const bool tiled = fits && g_prefill_f32_mfma != 2 &&
+                       (g_prefill_f32_mfma == 3 || per_row * (total_q / rows) >= 2 * cus);
     if (tiled) {
         const int nt = (max_seqlen_q + rows - 1) / rows;
         auto kern = head_dim == 64 ? (block_size == 16 ? prefill_f32_tile_kernel<64, true>
@@ -551,9 +554,14 @@ int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh
 
 using namespace flour;
 
-// 1 (the default): fp32 prefill at head_dim 64 / 128 on the fp32 matrix cores; 0: on the vector
-// kernel. A test / tuning switch.
-extern "C" int flour_hip_set_prefill_f32_mfma(int on) {
-    g_prefill_f32_mfma = on ? 1 : 0;
+// fp32 prefill at head_dim 64 / 128: 1 (the default) on the fp32 matrix cores, 0 on the vector
+// kernel; 2 and 3 as 1, but never / always, within its limits, on the tile kernel. A test / tuning
+// switch.
+extern "C" int flour_hip_set_prefill_f32_mfma(int mode) {
+    if (mode < 0 || mode > 3) {
+        set_error("set_prefill_f32_mfma: mode %d is not 0 to 3", mode);
+        return FLOUR_ERR_INVALID_ARGUMENT;
+    }
+    g_prefill_f32_mfma = mode;
     return FLOUR_OK;
 }

@@ -304,8 +304,10 @@ static int64_t thin_items(int slots, int num_seqs, int total_q, int num_heads, i
     return (int64_t)(num_heads / n_rep) * ((n_rep + hw - 1) / hw) * (total_q / rows + num_seqs);
 }
 
-// Whether a small batch runs here (varlen_prefill.hip's shape checks hold; `cus`: CUs of the
-// device), by its items at four slots. Measured against varlen_prefill.hip, us there / here, per
+// Slots per item of a small batch that runs here (varlen_prefill.hip's shape checks hold; `cus`: CUs
+// of the device), 0 where varlen_prefill.hip takes it: by its items at four slots, two slots up to
+// one item per CU (1 x 2,000 rows, 14 / 2 heads [252 items] 39.9 against 44.4 us, 8 x U[128, 512]
+// [352] 21.0 against 16.1). Measured against varlen_prefill.hip, us there / here, per
 // call from Python (~12 us at least), items in brackets:
 //   1 x 1,000 rows, 14 / 2 heads [128] 29.6 / 20.7; 1 x 2,000 [252] 51.2 / 39.9; 8 x U[128, 512]
 //   [352] 19.3 / 16.1; 8 / 8 heads, 1 x 2,000 [128] 50.2 / 32.5; 32 / 32 heads, 1 x 1,000 [256]
@@ -314,10 +316,14 @@ static int64_t thin_items(int slots, int num_seqs, int total_q, int num_heads, i
 // At head_dim 128 the same kernel was even (32 / 8 heads, 1 x 1,000 rows 39.9 / 39.3, 3 x U[64, 512]
 // 20.8 / 21.2; 1 x 2,000 74 / 79; only 1 x 256 gained, 17.0 / 15.6): a step there is bound by products
 // and the wider staging of fewer rows costs what the split gains.
-bool prefill_thin_wanted(int num_seqs, int max_seqlen_q, int total_q, int num_heads, int n_rep,
-                         int head_dim, int cus) {
-    return head_dim == PT_D && num_seqs <= 64 && max_seqlen_q <= 65536 &&
-           thin_items(4, num_seqs, total_q, num_heads, n_rep) <= cus + cus / 2;
+static int g_prefill_small = 1;  // a test / tuning switch
+
+int prefill_thin_slots(int num_seqs, int max_seqlen_q, int total_q, int num_heads, int n_rep,
+                       int head_dim, int cus) {
+    if (g_prefill_small == 0 || head_dim != PT_D || num_seqs > 64 || max_seqlen_q > 65536) return 0;
+    if (g_prefill_small > 1) return g_prefill_small;
+    const int64_t items = thin_items(4, num_seqs, total_q, num_heads, n_rep);
+    return items <= cus ? 2 : items <= cus + cus / 2 ? 4 : 0;
 }
 
 int launch_prefill_thin(int dtype, int out_dtype, void* out, int64_t o_st, int64_t o_sh,
@@ -325,12 +331,9 @@ int launch_prefill_thin(int dtype, int out_dtype, void* out, int64_t o_st, int64
                         const void* v_pool, const int32_t* cu, const int32_t* q_rows,
                         const int32_t* kv_lens, const int32_t* bt, int max_blocks, int num_seqs,
                         int max_seqlen_q, int total_q, int num_heads, int n_rep, int block_size,
-                        int64_t num_slots, float scale, int cus, bool persistent,
+                        int64_t num_slots, float scale, int slots, int cus, bool persistent,
                         hipStream_t stream) {
     const int kv_heads = num_heads / n_rep;
-    // two slots up to one item per CU at four (1 x 2,000 rows, 14 / 2 heads [252 items] 39.9 against
-    // 44.4 us, 8 x U[128, 512] [352] 21.0 against 16.1)
-    const int slots = thin_items(4, num_seqs, total_q, num_heads, n_rep) <= cus ? 2 : 4;
     const int hw = std::min(item_heads(n_rep), slots), rows = 32 * (slots / hw);
     const int n_qt = (max_seqlen_q + rows - 1) / rows;
     const int64_t items = thin_items(slots, num_seqs, total_q, num_heads, n_rep);
@@ -363,3 +366,17 @@ int launch_prefill_thin(int dtype, int out_dtype, void* out, int64_t o_st, int64
 }
 
 }  // namespace flour
+
+using namespace flour;
+
+// 16-bit prefill at head_dim 64: 1 (the default): small batches on this kernel, by the rule above;
+// 0: none; 2, 4: every batch of up to 64 sequences, with that many slots an item. A test / tuning
+// switch.
+extern "C" int flour_hip_set_prefill_small(int mode) {
+    if (mode != 0 && mode != 1 && mode != 2 && mode != 4) {
+        set_error("set_prefill_small: mode %d is not 0, 1, 2 or 4", mode);
+        return FLOUR_ERR_INVALID_ARGUMENT;
+    }
+    g_prefill_small = mode;
+    return FLOUR_OK;
+}

@@ -57,14 +57,14 @@ int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh
                             int num_seqs, int max_seqlen_q, int total_q, int num_heads, int n_rep,
                             int head_dim, int block_size, int64_t num_slots, float scale,
                             hipStream_t stream);
-bool prefill_thin_wanted(int num_seqs, int max_seqlen_q, int total_q, int num_heads, int n_rep,
-                         int head_dim, int cus);
+int prefill_thin_slots(int num_seqs, int max_seqlen_q, int total_q, int num_heads, int n_rep,
+                       int head_dim, int cus);
 int launch_prefill_thin(int dtype, int out_dtype, void* out, int64_t o_st, int64_t o_sh,
                         const void* q, int64_t q_st, int64_t q_sh, const void* k_pool,
                         const void* v_pool, const int32_t* cu, const int32_t* q_rows,
                         const int32_t* kv_lens, const int32_t* bt, int max_blocks, int num_seqs,
                         int max_seqlen_q, int total_q, int num_heads, int n_rep, int block_size,
-                        int64_t num_slots, float scale, int cus, bool persistent,
+                        int64_t num_slots, float scale, int slots, int cus, bool persistent,
                         hipStream_t stream);
 bool simt_supported(int dtype, int head_dim, const void* q, int64_t q_st, int64_t q_sh,
                     const void* k_pool, const void* v_pool);
@@ -1783,13 +1783,16 @@ static int varlen_prefill_impl(void* out, int out_dtype, int64_t o_stride_tok,
                                    scale, s);
     }
     // small batches at head_dim 64: more, shorter items
-    if (g_prefill_pv_mode == PV_F16 &&
-        prefill_thin_wanted(num_seqs, max_seqlen_q, total_q, num_heads, n_rep, head_dim, device_cus()))
+    const int slots = g_prefill_pv_mode == PV_F16
+                          ? prefill_thin_slots(num_seqs, max_seqlen_q, total_q, num_heads, n_rep,
+                                               head_dim, device_cus())
+                          : 0;
+    if (slots)
         return launch_prefill_thin(dtype, out_dtype, out, o_stride_tok, o_stride_head, q,
                                    q_stride_tok, q_stride_head, k_pool, v_pool, cu_seqlens_q,
                                    q_rows, kv_lens, block_tables, max_blocks_per_seq, num_seqs,
                                    max_seqlen_q, total_q, num_heads, n_rep, block_size, num_slots,
-                                   scale, device_cus(), g_prefill_persistent != 0, s);
+                                   scale, slots, device_cus(), g_prefill_persistent != 0, s);
 #define FLOUR_PF_D(T, TO, D)                                                                     \
     return g_prefill_pv_mode == PV_HILO                                                          \
                ? launch_prefill_mfma<T, TO, PV_HILO, D>(                                         \

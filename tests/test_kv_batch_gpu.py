@@ -180,15 +180,26 @@ def _fill(b, sids, lens, layer, seed):
         b.write_kv(layer, k, v)
 
 
-def test_mixed_step_runs_decode_rows_on_the_decode_kernel(device):
-    """A continuous-batching step at the Llama-3-8B attention shape: 60 sequences decoding one
+@pytest.fixture
+def small(request):
+    """Which prefill kernel head_dim-64 calls run on: 0 the large one, 2 / 4 the one for small
+    batches with that many slots an item, 1 the library's rule."""
+    assert _lib.lib().flour_hip_set_prefill_small(request.param) == 0
+    yield request.param
+    _lib.lib().flour_hip_set_prefill_small(1)
+
+
+@pytest.mark.parametrize("Hq,Gk,Dh,small", [(32, 8, 128, 1), (14, 2, 64, 0), (14, 2, 64, 2),
+                                            (14, 2, 64, 4)], indirect=["small"])
+def test_mixed_step_runs_decode_rows_on_the_decode_kernel(device, Hq, Gk, Dh, small):
+    """A continuous-batching step at the Llama-3-8B attention shape, and at Qwen2.5-0.5B's on each
+    form of the head_dim-64 prefill: 60 sequences decoding one
     row each over contexts U[512, 4096] while 4 prompts of U[128, 512] rows prefill, listed
     interleaved. The one-row sequences run as one paged-decode launch and the prompts as one
     prefill launch, each over its rows of the packed layout: every row against the oracle,
     the decode rows bit-identical to paged_decode over those sequences alone, the prompt rows
     bit-identical to varlen_prefill over the prompts alone, and the all-prefill route (the
     split switched off) against the oracle too."""
-    Hq, Gk, Dh = 32, 8, 128
     rng = np.random.default_rng(41)
     b = KvBatch(1, 10000, 64, 4096 + 16, 8 * 4096, Hq, Gk, Dh, torch.bfloat16, BS)
     n_dec = 60

@@ -1,13 +1,17 @@
-"""Causal varlen prefill at head_dim 64 on the matrix-core kernel (the Qwen2.5-0.5B attention
+"""Causal varlen prefill at head_dim 64 on the matrix-core kernels (the Qwen2.5-0.5B attention
 shape the reference serves: 14 q / 2 kv heads, GQA 7, src/models/qwen2.rs:39 with
 script/script.js:14), against the oracle's restatement of paged_attention (cpu.rs:57-112).
 
+Two kernels serve it: the large one (varlen_prefill.hip) and the one for small batches
+(prefill_thin.hip, with two or four slots an item). Every case that is small enough for either
+runs on all three forms, whatever the dispatch rule says for its size (`kernel`).
+
 Bounds as for head_dim 128: the fp32 accumulator output within max-abs 2e-3 and rel-L2 1e-3 of
 the fp32 oracle, the bf16 output within the ulp bounds of tests/_util.py. Covered: GQA 7, a
-cached prefix shared by every sequence, partial last query tiles (the 4 x 64 and 8 x 32 item
-shapes and the one-head 256-row items of an odd group), page sizes 16 and 32, kv_len < q_len,
-the persistent schedule against one workgroup per item, V outside the fp16 range (the exact
-redo), the hi + lo P mode and the whole benchmark batch.
+cached prefix shared by every sequence, partial last query tiles (the large kernel's 4 x 64 and 8 x
+32 item shapes and the one-head 256-row items of an odd group), page sizes 16, 32 and 48, kv_len <
+q_len, the persistent schedule against one workgroup per item, V outside the fp16 range (the large
+kernel's exact redo), the hi + lo P mode and the whole benchmark batch.
 """
 from __future__ import annotations
 
@@ -23,6 +27,14 @@ from test_prefill_gpu import oracle_prefill, run, write
 pytestmark = pytest.mark.gpu
 
 D = 64
+
+
+@pytest.fixture(params=[0, 2, 4], ids=["large", "two-slot", "four-slot"])
+def kernel(request):
+    """The kernel form that the test's calls run on."""
+    assert _lib.lib().flour_hip_set_prefill_small(request.param) == 0
+    yield request.param
+    _lib.lib().flour_hip_set_prefill_small(1)
 
 
 def check(c, seqs=None, tag=""):
@@ -60,14 +72,14 @@ def go(c, persistent=1, out_dtype=torch.float32):
     (8, 1, 16, [1, 200], 160),              # n_rep 8
     (14, 2, 48, [150, 96], 96),             # 48-token pages
 ])
-def test_prefill_d64_shapes(device, H, G, bs, lens, prefix):
+def test_prefill_d64_shapes(device, kernel, H, G, bs, lens, prefix):
     c = make_prefill(len(lens), H, G, D, bs, (1, 1), prefix=prefix, dtype=torch.bfloat16,
                      seed=H * 5 + G + bs, device=device, q_lens=lens)
     write(c)
     check(c, tag=f"D64 H={H} G={G} bs={bs} lens={lens} prefix={prefix}")
 
 
-def test_prefill_d64_f16_pools(device):
+def test_prefill_d64_f16_pools(device, kernel):
     c = make_prefill(3, 14, 2, D, 16, (1, 1), prefix=32, dtype=torch.float16, seed=61,
                      device=device, q_lens=[200, 64, 9])
     write(c)
@@ -110,9 +122,10 @@ def test_prefill_d64_persistent_and_partial_tiles(device, H, G):
     assert max_abs <= 2e-3 and rel <= 1e-3
 
 
-def test_prefill_d64_v_outside_fp16_range(device):
-    """V rows of +-1e5 and 1e-30 among N(0,1) rows: the items that meet them are recomputed in
-    exact mode (bf16 V, P split in two); judged against the output's own scale."""
+def test_prefill_d64_v_outside_fp16_range(device, kernel):
+    """V rows of +-1e5 and 1e-30 among N(0,1) rows: the large kernel recomputes the items that meet
+    them in exact mode (bf16 V, P split in two), the small-batch kernel always keeps V in bf16 and P
+    in two parts; judged against the output's own scale."""
     c = make_prefill(4, 14, 2, D, 16, (1, 1), prefix=32, dtype=torch.bfloat16, seed=81,
                      device=device, q_lens=[150, 40, 260, 7])
     c.v_new[10:14] *= 1e5
@@ -139,7 +152,7 @@ def test_prefill_d64_hilo_mode(device):
     assert np.isfinite(got).all()
 
 
-def test_prefill_d64_reference_layout(device):
+def test_prefill_d64_reference_layout(device, kernel):
     """q in the reference's head-major (1, heads, seq, D) layout and out written straight into
     (seq, heads, D): strided views on both sides."""
     c = make_prefill(1, 14, 2, D, 16, (1, 1), prefix=0, dtype=torch.bfloat16, seed=95,
@@ -156,18 +169,19 @@ def test_prefill_d64_reference_layout(device):
 
 
 @pytest.mark.parametrize("H,G,bs,lens,prefix,short", [
-    (14, 2, 16, [1000], 0, None),                     # one prompt, two slots an item (GQA 7)
-    (14, 2, 16, [511, 130, 64, 33, 1, 385, 500, 480], 0, 3),  # four slots, row and step edges
+    (14, 2, 16, [1000], 0, None),                     # one prompt, GQA 7
+    (14, 2, 16, [511, 130, 64, 33, 1, 385, 500, 480], 0, 3),  # row and step edges
     (8, 8, 32, [129, 128, 1, 65], 32, None),          # one head an item, 32-token pages
     (6, 2, 48, [200, 31], 96, 1),                     # n_rep 3, 48-token pages
     (16, 1, 16, [40] * 64, 256, 7),                   # n_rep 16, 64 sequences
+    (4, 2, 32, [1, 63, 64, 65, 129], 0, 2),           # n_rep 2: both heads, one or two row blocks
     (12, 2, 16, [300], 1008, None),                   # n_rep 6, a prefix that ends inside a step
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_small_batches(device, dtype, H, G, bs, lens, prefix, short):
-    """Batches small enough for the 32-row items: against the oracle, with garbage in every row past
-    the sequences' positions, bad block ids past the used pages, a sequence whose kv length is below
-    its query count, and both schedules alike."""
+def test_small_batches(device, kernel, dtype, H, G, bs, lens, prefix, short):
+    """Batches of the small-batch kernel's sizes on each form: against the oracle, with garbage in
+    every row past the sequences' positions, bad block ids past the used pages, a sequence whose kv
+    length is below its query count, and both schedules alike."""
     c = make_prefill(len(lens), H, G, D, bs, (1, 1), prefix=prefix, dtype=dtype, seed=H + bs,
                      device=device, q_lens=lens)  # (every pool row is filled)
     used = torch.zeros(c.k_pool.shape[1], dtype=torch.bool)
@@ -192,7 +206,7 @@ def test_small_batches(device, dtype, H, G, bs, lens, prefix, short):
 
 
 @pytest.mark.parametrize("bound", [1000, 1024, 40000, 65536])
-def test_small_batch_with_a_loose_row_bound(device, bound):
+def test_small_batch_with_a_loose_row_bound(device, kernel, bound):
     """max_seqlen_q is a bound: one far above the longest sequence changes nothing."""
     c = make_prefill(3, 14, 2, D, 16, (1, 1), prefix=32, dtype=torch.bfloat16, seed=97,
                      device=device, q_lens=[400, 64, 9])

@@ -56,6 +56,14 @@ def test_prefill_f32_matrix_cores_match_oracle(device, H, G, D, bs, lens, prefix
     assert max_abs <= 1e-5
 
 
+@pytest.fixture
+def tiles():
+    """fp32 prefill on the tile kernel, whatever the dispatch rule says for the batch."""
+    assert _lib.lib().flour_hip_set_prefill_f32_mfma(3) == 0
+    yield
+    _lib.lib().flour_hip_set_prefill_f32_mfma(1)
+
+
 @pytest.mark.parametrize("H,G,D,bs,lens,prefix,short", [
     (128, 128, 64, 16, [129, 1, 127, 260], 0, None),         # n_rep 1: 128-row items, their edges
     (128, 64, 128, 32, [64, 65, 1, 63, 200, 130], 32, 3),    # n_rep 2: 64-row items, 32-token pages
@@ -64,8 +72,8 @@ def test_prefill_f32_matrix_cores_match_oracle(device, H, G, D, bs, lens, prefix
     (96, 32, 128, 16, [680, 100], 0, None),                  # n_rep 3: one head an item
     (64, 16, 64, 16, [17] * 64, 128, 40),                    # 64 sequences
 ])
-def test_prefill_f32_tiles_match_oracle(device, H, G, D, bs, lens, prefix, short):
-    """Batches of two items per CU or more (the tile kernel): against the oracle, with rows past
+def test_prefill_f32_tiles_match_oracle(device, tiles, H, G, D, bs, lens, prefix, short):
+    """The tile kernel (larger batches): against the oracle, with rows past
     each sequence's positions holding garbage, a sequence whose kv length is below its query count,
     a bad block id past the used pages and 16-bit outputs."""
     c = make_prefill(len(lens), H, G, D, bs, (1, 1), prefix=prefix, dtype=torch.float32,
@@ -91,7 +99,7 @@ def test_prefill_f32_tiles_match_oracle(device, H, G, D, bs, lens, prefix, short
 
 
 @pytest.mark.parametrize("bound", [700, 20000, 1 << 20])
-def test_prefill_f32_tiles_with_a_loose_row_bound(device, bound):
+def test_prefill_f32_tiles_with_a_loose_row_bound(device, tiles, bound):
     """max_seqlen_q is a bound: one far above the longest sequence changes nothing."""
     c = make_prefill(4, 64, 16, 128, 16, (1, 1), prefix=0, dtype=torch.float32, seed=98,
                      device="cuda:0", q_lens=[680, 600, 1, 300])
