@@ -1168,12 +1168,23 @@ static bool decode_f32_split(int head_dim, int block_size, int n_rep, int batch,
     // two) x head_dim; a split step takes ~9 us and its bytes. Vector / split in us: 1 x 256 tokens of
     // 32 / 8 heads of 128 14.5 / 10.3 (64 tokens: 7.4 / 9.8), 14 / 2 heads of 64 13.4 / 8.8 (64: 8.3 /
     // 8.4), 16 / 16 of 128 at 1,024 18.3 / 11.8 (256: 7.7 / 10.2), 8 / 8 of 64 at 2,048 19.9 / 10.0
-    // (512: 8.1 / 9.0). At n_rep 1 with one full round of workgroups the vector kernel is better
-    // for as long again: 16 x 8 / 8 heads of 64 at 2,048 23.8 / 26.3, at 8,192 102 / 79.
-    int64_t work = (int64_t)max_context_len * head_dim;
-    for (int nq = 1; nq < n_rep && nq < 8; nq *= 2) work *= 2;
-    const int64_t pairs = (int64_t)batch * num_heads / n_rep;
-    return work >= (n_rep == 1 && pairs >= 128 && pairs <= 256 ? 262144 : 131072);
+    // (512: 8.1 / 9.0).
+    int64_t work = (int64_t)max_context_len * head_dim, least = 131072;
+    int nq = 1;
+    for (; nq < n_rep && nq < 8; nq *= 2) work *= 2;
+    // With few queries per row and a workgroup for most CUs the vector kernel reads at HBM's rate too.
+    // Up to one per CU all of them end together, and at one or two queries the split kernel is the
+    // slower one at any length (16 / 16 heads of 64, 12 x 4,096 tokens: 73 / 80; 32 / 16 of 64, 12 x
+    // 2,149: 38 / 49; 16 x 4,096 of 16 / 16 heads 99 / 91); otherwise it needs a longer step for its
+    // 9 us (12 / 4 of 64, 128 x 512 tokens: 29 / 31, x 1,024 55 / 53; 16 / 8 of 128, 64 x 512: 46 /
+    // 50, x 1,024 105 / 93). Over 26,379 batches of 16-1,200 (sequence, kv head) pairs, lengths uniform
+    // and ragged, the step taken is up to 7 times as fast as the vector kernel's and 3-8% slower in 10.
+    const int64_t pairs = (int64_t)batch * num_heads / n_rep, cus = device_cus();
+    if (nq == 1 ? 8 * pairs >= 3 * cus : 2 * pairs >= cus) {
+        if (nq <= 2 && 2 * pairs >= cus && pairs < cus) return false;
+        if (nq < 8 || pairs < cus) least *= 2;
+    }
+    return work >= least;
 }
 
 static int paged_decode_impl(void* out, int out_dtype, const void* q, const void* k_pool,

@@ -110,6 +110,42 @@ def test_decode_fp32_split(device, H, G, D, bs, ctx):
         assert torch.equal(run(c, dt), got.to(dt))
 
 
+@pytest.mark.parametrize("H,G,D,per_cu,tokens,split", [
+    # (sequence, kv head) pairs per CU; context length; whether the step is split
+    (8, 8, 64, 0, 2048, True), (8, 8, 64, 0, 2032, False),       # few pairs: from ctx x D x queries
+    (14, 2, 64, 0, 256, True), (14, 2, 64, 0, 240, False),       # of 131,072
+    (16, 16, 64, 5 / 16, 2048, True), (16, 16, 64, 6 / 16, 2048, False),  # one query: 3/8 of the CUs,
+    (16, 16, 64, 7 / 16, 4096, True),                            # then twice as long,
+    (16, 16, 64, 0.5, 8192, False), (16, 16, 64, 15 / 16, 8192, False),   # never from 1/2
+    (16, 16, 64, 1.0, 4096, True), (16, 16, 64, 1.0, 4080, False),     # to one per CU
+    (16, 8, 64, 15 / 32, 1024, True), (16, 8, 64, 0.5, 4096, False),  # two queries
+    (16, 8, 64, 1.0, 2048, True), (16, 8, 64, 1.0, 2032, False),
+    (16, 4, 64, 0.5, 1024, True), (16, 4, 64, 0.5, 1008, False),   # four
+    (14, 2, 64, 0.5, 512, True), (14, 2, 64, 0.5, 496, False), (14, 2, 64, 1.0, 256, True),  # eight
+])
+def test_decode_fp32_rule(device, H, G, D, per_cu, tokens, split):
+    """Which fp32 steps are split, on both sides of every line of the rule, told by the rounding: a
+    step on the vector kernel equals one without a workspace bit for bit. Sequences share pages."""
+    from flour_amd import _lib
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    B = max(1, int(per_cu * cus) // G)
+    g = torch.Generator(device=device).manual_seed(tokens + B)
+    pools = [torch.randn((G, 8192, D), generator=g, device=device) for _ in range(2)]
+    q = torch.randn((B, H, D), generator=g, device=device)
+    bt = torch.arange(tokens // 16, dtype=torch.int32, device=device).repeat(B, 1)
+    ctx = torch.full((B,), tokens, dtype=torch.int32, device=device)
+    ctx[B // 2] = max(1, tokens // 3)
+    vec = torch.empty_like(q)
+    p = ops._ptr
+    _lib.check(_lib.lib().flour_hip_paged_decode(
+        p(vec), 0, p(q), p(pools[0]), p(pools[1]), p(bt), bt.shape[1], p(ctx), B, H, G, D, 16, 8192,
+        tokens, D ** -0.5, 0, None, 0, ops._stream()))
+    got = ops.paged_decode(q, *pools, bt, ctx, D ** -0.5, tokens)
+    torch.cuda.synchronize()
+    assert torch.equal(got, vec) != split
+    assert errors(to_np(got), to_np(vec))[0] <= 1e-5
+
+
 def test_decode_fp32_split_on_two_streams(device):
     """fp32 steps without a workspace argument share none: overlapping calls on two streams give
     what each gives alone."""
