@@ -305,25 +305,30 @@ static int64_t thin_items(int slots, int num_seqs, int total_q, int num_heads, i
 }
 
 // Slots per item of a small batch that runs here (varlen_prefill.hip's shape checks hold; `cus`: CUs
-// of the device), 0 where varlen_prefill.hip takes it: by its items at four slots, two slots up to
-// one item per CU (1 x 2,000 rows, 14 / 2 heads [252 items] 39.9 against 44.4 us, 8 x U[128, 512]
-// [352] 21.0 against 16.1). Measured against varlen_prefill.hip, us there / here, per
-// call from Python (~12 us at least), items in brackets:
-//   1 x 1,000 rows, 14 / 2 heads [128] 29.6 / 20.7; 1 x 2,000 [252] 51.2 / 39.9; 8 x U[128, 512]
-//   [352] 19.3 / 16.1; 8 / 8 heads, 1 x 2,000 [128] 50.2 / 32.5; 32 / 32 heads, 1 x 1,000 [256]
-//   29.5 / 24.0, 3 x U[64, 512] [288] 17.6 / 13.3, 1 x 2,000 [512] 52.5 / 49.6, 8 x U[128, 512] [896]
-//   24.3 / 27.5; 8 / 8 heads, 16 x U[128, 512] behind a 1,024-token prefix [448] 42 / 57.
+// of the device), 0 where varlen_prefill.hip takes it. Over a long cached prefix all items are alike,
+// and a batch takes items per CU, rounded up, times ~12 ns a position with two slots and ~18 with
+// four, where varlen_prefill.hip's larger items take ~20 and are fewer: two slots up to one item per
+// CU, then four up to one, whatever the kv lengths. us there / here: 14 / 2 heads, 1 x 1,000 rows 29.6
+// / 20.7, 1 x 2,000 51.2 / 44.4; 8 / 8 heads, 1 x 2,000 50.2 / 32.5; 32 / 32, 3 x U[64, 512] 17.6 /
+// 13.3; 32 / 8, 4 x 191 behind 4,096 tokens 95 / 79; past that line 14 / 2, 16 x U[64, 286] behind
+// 1,024 35 / 47. A single prompt without a prefix (by the width of its block table) has items of every
+// length, which the snake pairs: two slots up to one item per CU at four (1 x 2,000 rows 39.9 against
+// 44.4 with four), four up to one and a half (1 x 2,867 rows 66.7 there, 58.8 here). Of
+// 21,794 batches of 1-64 sequences behind 0-4,096 tokens one is more than 3% slower than there (4%).
 // At head_dim 128 the same kernel was even (32 / 8 heads, 1 x 1,000 rows 39.9 / 39.3, 3 x U[64, 512]
-// 20.8 / 21.2; 1 x 2,000 74 / 79; only 1 x 256 gained, 17.0 / 15.6): a step there is bound by products
-// and the wider staging of fewer rows costs what the split gains.
+// 20.8 / 21.2; 1 x 2,000 74 / 79; only 1 x 256 gained, 17.0 / 15.6).
 static int g_prefill_small = 1;  // a test / tuning switch
 
-int prefill_thin_slots(int num_seqs, int max_seqlen_q, int total_q, int num_heads, int n_rep,
-                       int head_dim, int cus) {
+// kv_cap: the positions that a row of the block table holds.
+int prefill_thin_slots(int num_seqs, int max_seqlen_q, int total_q, int64_t kv_cap, int num_heads,
+                       int n_rep, int head_dim, int cus) {
     if (g_prefill_small == 0 || head_dim != PT_D || num_seqs > 64 || max_seqlen_q > 65536) return 0;
     if (g_prefill_small > 1) return g_prefill_small;
+    if (thin_items(2, num_seqs, total_q, num_heads, n_rep) <= cus) return 2;
     const int64_t items = thin_items(4, num_seqs, total_q, num_heads, n_rep);
-    return items <= cus ? 2 : items <= cus + cus / 2 ? 4 : 0;
+    if (num_seqs == 1 && kv_cap <= (int64_t)total_q + 256)
+        return items <= cus ? 2 : items <= cus + cus / 2 ? 4 : 0;
+    return items <= cus ? 4 : 0;
 }
 
 int launch_prefill_thin(int dtype, int out_dtype, void* out, int64_t o_st, int64_t o_sh,

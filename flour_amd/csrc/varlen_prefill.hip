@@ -57,8 +57,8 @@ int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh
                             int num_seqs, int max_seqlen_q, int total_q, int num_heads, int n_rep,
                             int head_dim, int block_size, int64_t num_slots, float scale,
                             hipStream_t stream);
-int prefill_thin_slots(int num_seqs, int max_seqlen_q, int total_q, int num_heads, int n_rep,
-                       int head_dim, int cus);
+int prefill_thin_slots(int num_seqs, int max_seqlen_q, int total_q, int64_t kv_cap, int num_heads,
+                       int n_rep, int head_dim, int cus);
 int launch_prefill_thin(int dtype, int out_dtype, void* out, int64_t o_st, int64_t o_sh,
                         const void* q, int64_t q_st, int64_t q_sh, const void* k_pool,
                         const void* v_pool, const int32_t* cu, const int32_t* q_rows,
@@ -1784,8 +1784,9 @@ static int varlen_prefill_impl(void* out, int out_dtype, int64_t o_stride_tok,
     }
     // small batches at head_dim 64: more, shorter items
     const int slots = g_prefill_pv_mode == PV_F16
-                          ? prefill_thin_slots(num_seqs, max_seqlen_q, total_q, num_heads, n_rep,
-                                               head_dim, device_cus())
+                          ? prefill_thin_slots(num_seqs, max_seqlen_q, total_q,
+                                               (int64_t)max_blocks_per_seq * block_size, num_heads,
+                                               n_rep, head_dim, device_cus())
                           : 0;
     if (slots)
         return launch_prefill_thin(dtype, out_dtype, out, o_stride_tok, o_stride_head, q,

@@ -213,3 +213,37 @@ def test_small_batch_with_a_loose_row_bound(device, kernel, bound):
     tight = go(c)
     c.max_seqlen_q = bound
     assert torch.equal(go(c), tight)
+
+
+@pytest.mark.parametrize("H,G,lens,prefix,slots", [
+    (14, 2, [31 * 32], 0, 2), (14, 2, [31 * 32], 4096, 2),  # 256 items with two slots each: one a CU
+    (14, 2, [32 * 32], 4096, 4),                            # 264 and 132: four slots
+    (14, 2, [63 * 32], 4096, 4), (14, 2, [64 * 32], 4096, 0),      # up to one a CU
+    (14, 2, [32 * 32], 0, 2), (14, 2, [63 * 32], 0, 2),     # one prompt without a prefix: two slots
+    (14, 2, [64 * 32], 0, 4), (14, 2, [95 * 32], 0, 4),     # there, four up to one and a half
+    (14, 2, [96 * 32], 0, 0),
+    (8, 8, [64 * 7] * 4, 0, 2), (8, 8, [64 * 8] * 4, 0, 4),      # one head an item
+    (32, 8, [32 * 3] * 8, 0, 4), (32, 8, [32 * 3 + 4] * 8, 0, 0),
+    (2, 2, [20] * 64, 256, 2), (2, 2, [20] * 65, 256, 0),   # up to 64 sequences
+])
+def test_small_batch_rule(device, H, G, lens, prefix, slots):
+    """Which batches run on the small-batch kernel and with how many slots, on both sides of every
+    line of the rule, told by the bits of the output."""
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    if cus != 256:
+        pytest.skip("the sizes are those of 256 CUs")
+    c = make_prefill(len(lens), H, G, D, 16, (1, 1), prefix=prefix, dtype=torch.bfloat16,
+                     seed=len(lens), device=device, q_lens=lens)
+    got = go(c)
+    lib = _lib.lib()
+    same = []
+    try:
+        for mode in (0, 2, 4):
+            lib.flour_hip_set_prefill_small(mode)
+            out = go(c)
+            assert errors(to_np(out), to_np(got))[1] <= 1e-3
+            if torch.equal(out, got):
+                same.append(mode)
+    finally:
+        lib.flour_hip_set_prefill_small(1)
+    assert same == [slots] if len(lens) <= 64 else slots in same
