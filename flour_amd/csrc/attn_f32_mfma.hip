@@ -260,6 +260,7 @@ __global__ __launch_bounds__(F32T_WAVES * 64, 2) void prefill_f32_tile_kernel(
     constexpr int NS = 16 * DT + 2;           // a lane's state: O^T registers, max, sum
     __shared__ __attribute__((aligned(16))) float lds[4 * KT * D];
     static_assert(4 * (F32T_SPLIT - 1) * NS * 64 <= 4 * KT * D, "the states fit the tiles");
+    __shared__ ItemSeq seqs[64];
     auto kt = [&](int buf) { return lds + buf * KT * D; };
     auto vt = [&](int buf) { return lds + (2 + buf) * KT * D; };
 
@@ -272,17 +273,20 @@ __global__ __launch_bounds__(F32T_WAVES * 64, 2) void prefill_f32_tile_kernel(
     const uint32_t head_bytes = (uint32_t)num_slots * D * 4u;
     const int G = gridDim.x;
 
-    ItemWalk items;
-    items.start(cu_seqlens_q, kv_lens, num_seqs, max_blocks * block_size, rows, n_qt, per_row, lane);
+    using Walk = ItemWalk<true>;
+    Walk items;
+    items.start(cu_seqlens_q, kv_lens, num_seqs, max_blocks * block_size, rows, n_qt, per_row, lane,
+                seqs);
     if (ks == 0) __builtin_amdgcn_s_setprio(1);
 
     for (int round = 0;; round++) {
         int s, qt, x;
-        if (!items.find(ItemWalk::deal(round, G, blockIdx.x), lane, s, qt, x)) break;
+        ItemSeq sq;
+        if (!items.find(Walk::deal(round, G, blockIdx.x), lane, s, sq, qt, x)) break;
         const int kvh = x / groups, h0 = (x - kvh * groups) * hw;
-        const int c0 = __builtin_amdgcn_readlane(items.c0, s);
-        const int q_len = __builtin_amdgcn_readlane(items.rows, s);
-        const int kv_len = __builtin_amdgcn_readlane(items.kv, s);
+        const int c0 = sq.c0;
+        const int q_len = sq.rows;
+        const int kv_len = sq.kv;
         const int off = kv_len - q_len;  // row i sees positions j <= off + i
         const bool reads = kv_len >= q_len;
         const int kv_end = reads ? off + min(qt * rows + rows, q_len) : 0;  // the item's range

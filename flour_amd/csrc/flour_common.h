@@ -246,6 +246,15 @@ __device__ __forceinline__ float wave_max(float x) {
     x = fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xf, 0xf, false)));
     return max_across_rows(x);
 }
+// Maximum over all 64 lanes as a scalar: DPP row rotations, then the four rows' lanes 0.
+__device__ __forceinline__ int wave_max_i32(int x) {
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x124, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x122, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x121, 0xf, 0xf, false));
+    return max(max(__builtin_amdgcn_readlane(x, 0), __builtin_amdgcn_readlane(x, 16)),
+               max(__builtin_amdgcn_readlane(x, 32), __builtin_amdgcn_readlane(x, 48)));
+}
 // x + x of lane l^32 with one row swap (VALU) instead of an LDS permute.
 __device__ __forceinline__ float sum_across_halves(float x) {
     const uint32_t u = __float_as_uint(x);

@@ -76,16 +76,18 @@ __global__ __launch_bounds__(PT_WAVES * 64, 2) void prefill_thin_kernel(
     const int v_tp = tid % RPP, v_col = (tid / RPP) * 8;
     auto sigma16 = [](int t) { return (t & ~12) | ((t & 4) << 1) | ((t & 8) >> 1); };
 
-    ItemWalk items;
+    using Walk = ItemWalk<false>;
+    Walk items;
     items.start(cu_seqlens, kv_lens, num_seqs, max_blocks * block_size, rows, n_qt,
                 kv_heads * groups, lane);
     for (int round = 0;; round++) {
         int s, qt, x;
-        if (!items.find(ItemWalk::deal(round, gridDim.x, blockIdx.x), lane, s, qt, x)) break;
+        ItemSeq sq;
+        if (!items.find(Walk::deal(round, gridDim.x, blockIdx.x), lane, s, sq, qt, x)) break;
         const int kvh = x / groups, h0 = (x - kvh * groups) * hw;
-        const int c0 = __builtin_amdgcn_readlane(items.c0, s);
-        const int q_len = __builtin_amdgcn_readlane(items.rows, s);
-        const int kv_len = __builtin_amdgcn_readlane(items.kv, s);
+        const int c0 = sq.c0;
+        const int q_len = sq.rows;
+        const int kv_len = sq.kv;
         const int row0 = q_rows ? __builtin_amdgcn_readfirstlane(q_rows[s]) : c0;
         const int off = kv_len - q_len;  // row i sees positions j <= off + i
         const bool reads = kv_len >= q_len;

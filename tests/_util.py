@@ -85,3 +85,15 @@ def check_bf16_output(got_bits: np.ndarray, got32: np.ndarray, ref: np.ndarray,
         assert max_ulp_above(got_bits, ref, e) <= n, (f"more than {n} bf16 ulps from "
                                                       f"RNE(reference) where |ref| >= 2^{e}", rep)
     return rep
+
+
+def with_kv_lens(c, kv_lens: list[int], seed: int = 0):
+    """Gives each sequence of a prefill case its own kv length (its rows stay the last ones), over
+    pages drawn from the whole pool (sequences may share some)."""
+    blocks = c.k_pool.shape[1] // c.block_size
+    width = (max(kv_lens) + c.block_size - 1) // c.block_size
+    g = torch.Generator().manual_seed(seed)
+    c.block_tables = torch.randint(0, blocks, (len(kv_lens), width), generator=g,
+                                   dtype=torch.int32).to(c.q.device)
+    c.kv_lens = torch.tensor(kv_lens, dtype=torch.int32, device=c.q.device)
+    return c

@@ -19,7 +19,7 @@ import numpy as np
 import pytest
 import torch
 
-from _util import PREFILL_ULP_BOUNDS, check_bf16_output, errors, to_np
+from _util import PREFILL_ULP_BOUNDS, check_bf16_output, errors, to_np, with_kv_lens
 from flour_amd import _lib, ops
 from flour_amd.workloads import make_prefill, make_workload
 from test_prefill_gpu import oracle_prefill, run, write
@@ -247,3 +247,18 @@ def test_small_batch_rule(device, H, G, lens, prefix, slots):
     finally:
         lib.flour_hip_set_prefill_small(1)
     assert same == [slots] if len(lens) <= 64 else slots in same
+
+
+def test_prefixes_of_every_length(device, kernel):
+    """Sequences behind cached prefixes of their own lengths, far apart and none, in one batch: every
+    tile of each once, on every row, in both schedules."""
+    lens = [33, 1, 300, 64, 0, 128, 40, 257, 16, 96]
+    kv = [33, 4001, 300, 2064, 0, 128 + 31, 39, 257 + 640, 1016, 96 + 33]  # one below its rows
+    c = with_kv_lens(make_prefill(len(lens), 14, 2, D, 16, (1, 1), dtype=torch.bfloat16, seed=99,
+                                  device=device, q_lens=lens), kv)
+    got = go(c)
+    ref, rows = oracle_prefill(c)
+    max_abs, rel = errors(to_np(got)[rows], ref)
+    print(f"D64 ragged prefixes: max_abs={max_abs:.3e} rel_l2={rel:.3e}", flush=True)
+    assert max_abs <= 2e-3 and rel <= 1e-3
+    assert torch.equal(got, go(c, persistent=0))

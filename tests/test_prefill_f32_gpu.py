@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import oracle as O
-from _util import errors, f32_to_bf16_bits, to_np
+from _util import errors, f32_to_bf16_bits, to_np, with_kv_lens
 from flour_amd import _lib, ops
 from flour_amd.workloads import make_prefill, make_workload
 
@@ -96,6 +96,21 @@ def test_prefill_f32_tiles_match_oracle(device, tiles, H, G, D, bs, lens, prefix
         assert not got[a:b].any()
     for dt in (torch.bfloat16, torch.float16):
         assert torch.equal(_run(c, dt), got.to(dt))
+
+
+@pytest.mark.parametrize("H,G,D", [(8, 8, 64), (32, 16, 128), (14, 2, 64), (64, 16, 128)])
+def test_prefill_f32_tiles_prefixes_of_every_length(device, tiles, H, G, D):
+    """Sequences behind cached prefixes of their own lengths, far apart and none, in one batch: every
+    tile of each once, against the oracle on every row."""
+    lens = [33, 1, 300, 64, 0, 128, 40, 257, 16, 96]
+    kv = [33, 4001, 300, 2064, 0, 128 + 31, 39, 257 + 640, 1016, 96 + 33]  # one below its rows
+    c = with_kv_lens(make_prefill(len(lens), H, G, D, 16, (1, 1), dtype=torch.float32, seed=D + H,
+                                  device="cuda:0", q_lens=lens), kv)
+    out = torch.full_like(c.q, 7.0)
+    _run(c, out=out)
+    max_abs, _ = errors(to_np(out), _oracle(c))
+    print(f"fp32 ragged prefixes H={H} G={G} D={D}: max_abs={max_abs:.3e}", flush=True)
+    assert max_abs <= 1e-5
 
 
 @pytest.mark.parametrize("bound", [700, 20000, 1 << 20])
