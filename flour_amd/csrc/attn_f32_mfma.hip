@@ -514,11 +514,19 @@ int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh
     if (n_qt == 0 || num_seqs == 0) return FLOUR_OK;
     const dim3 grid((unsigned)num_heads, (unsigned)num_seqs, (unsigned)n_qt);
     const float sl2 = scale * 1.4426950408889634f;
-    // The tile kernel from two full-tile items per CU on (item tiles counted from the batch's rows):
-    // with fewer, an item's chain of steps bounds it, which the other kernel splits over 4 or 8
-    // waves. Measured, other / tile in us: 32 / 8 heads of 128, 1 x 1,024 rows (1 item per CU) 120 /
-    // 157, 2 x 1,024 203 / 168; 8 / 8 of 64, 1 x 1,024 (1/4) 29 / 77, 8 x 1,024 (2) 123 / 102; 16 /
-    // 16 of 128, 4 x U[512, 1,024] (1.5) 130 / 136; 14 / 2 of 64, 8 x U[256, 1,024] (2.5) 113 / 114.
+    // Which batches run on the tile kernel. Its items are larger and split over two waves instead of
+    // four or eight, so it needs enough of them, none that outlasts the rest, and full ones. Measured,
+    // other / tile in us:
+    //  * Items per CU, counted from the batch's rows: 32 / 8 heads of 128, 1 x 1,024 rows (1) 120 /
+    //    157, 2 x 1,024 (2) 203 / 168; 14 / 2 of 64, whose groups of four leave a slot without a head,
+    //    1 x 6,190 (3.0) 697 / 758. From 2.5, 4 with such a slot or with 128-row items.
+    //  * Rows per sequence: 16 / 16 of 128 (128-row items), 32 x 132 rows 94 / 143, 32 x 324 325 / 354,
+    //    8 x 1,296 848 / 742. At least 64, 128 and 640.
+    //  * The longest item that the block table allows, which the host cannot tell from a cached prefix
+    //    of all: up to 1.5 times a CU's share of the rows' own causal ranges. 28 / 4 of 128, 64 x 42
+    //    rows, one behind 4,096 tokens 308 / 610; 32 / 8 of 128, 1 x 2,075 behind 2,048 1,096 / 1,175.
+    // Of 21,095 batches with and without prefixes, some of one sequence alone, this takes 7,337: 7 of
+    // them are more than 3% slower than on the other kernel, the geometric mean is 1.24x.
     // Its item list holds up to 64 sequences, its loads 32-bit offsets.
     const int hw = item_heads(n_rep), kv_heads = num_heads / n_rep;
     const int rows = F32M_QT * (4 / hw);
@@ -526,8 +534,15 @@ int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh
     const int64_t cus = device_cus_f32();
     const bool fits = !q_rows && num_seqs <= 64 && num_slots * head_dim * 4 <= 0x7fffffff &&
                       per_row * num_seqs * ((int64_t)max_seqlen_q / rows + 1) <= 0x3fffffff;
-    const bool tiled = fits && g_prefill_f32_mfma != 2 &&
-                       (g_prefill_f32_mfma == 3 || per_row * (total_q / rows) >= 2 * cus);
+    const int64_t full = per_row * (total_q / rows);  // items of full tiles
+    const bool spare = n_rep % hw != 0;               // slots without a head
+    const int mean = total_q / num_seqs;
+    const int64_t kv_cap = (int64_t)max_blocks * block_size;
+    const bool wanted = 2 * full >= (spare || rows == 128 ? 8 : 5) * cus &&
+                        mean >= (rows == 128 ? 640 : spare ? 128 : 64) &&
+                        4 * kv_cap * cus <= 3 * full * mean;
+    const bool tiled =
+        fits && g_prefill_f32_mfma != 2 && (g_prefill_f32_mfma == 3 || wanted);
     if (tiled) {
         const int nt = (max_seqlen_q + rows - 1) / rows;
         auto kern = head_dim == 64 ? (block_size == 16 ? prefill_f32_tile_kernel<64, true>

@@ -123,6 +123,38 @@ def test_prefill_f32_tiles_with_a_loose_row_bound(device, tiles, bound):
     assert torch.equal(_run(c), tight)
 
 
+@pytest.mark.parametrize("H,G,D,lens,width,tiled", [
+    # block table width in positions (0: the longest sequence's)
+    (32, 8, 128, [640] * 4, 0, True), (32, 8, 128, [632] * 4, 0, False),   # 2.5 items per CU
+    (32, 8, 128, [64] * 40, 0, True), (32, 8, 128, [62] * 60, 0, False),   # 64 rows each
+    (28, 4, 128, [1024] * 4, 0, True), (28, 4, 128, [1016] * 4, 0, False),  # a spare slot: 4 per CU
+    (28, 4, 128, [128] * 32, 0, True), (28, 4, 128, [126] * 50, 0, False),  # and 128 rows each
+    (16, 16, 128, [1024] * 8, 0, True), (16, 16, 128, [1016] * 8, 0, False),  # 128-row items
+    (16, 16, 128, [640] * 13, 0, True), (16, 16, 128, [632] * 15, 0, False),  # and 640 rows each
+    (32, 8, 128, [640] * 4, 1200, True), (32, 8, 128, [640] * 4, 1216, False),  # room for a prefix:
+])                                                                       # 0.75 x 2.5 x 640 positions
+def test_prefill_f32_tile_rule(device, H, G, D, lens, width, tiled):
+    """Which fp32 batches run on the tile kernel, on both sides of every line of the rule, told by
+    the bits of the output."""
+    if torch.cuda.get_device_properties(device).multi_processor_count != 256:
+        pytest.skip("the sizes are those of 256 CUs")
+    c = make_prefill(len(lens), H, G, D, 16, (1, 1), dtype=torch.float32, seed=len(lens),
+                     device="cuda:0", q_lens=lens)
+    if width:
+        c.block_tables = torch.nn.functional.pad(c.block_tables,
+                                                 (0, width // 16 - c.block_tables.shape[1]))
+    got = _run(c)
+    outs = []
+    try:
+        for mode in (2, 3):
+            assert _lib.lib().flour_hip_set_prefill_f32_mfma(mode) == 0
+            outs.append(_run(c))
+    finally:
+        _lib.lib().flour_hip_set_prefill_f32_mfma(1)
+    assert errors(to_np(outs[0]), to_np(outs[1]))[0] <= 2e-5
+    assert torch.equal(got, outs[tiled]) and not torch.equal(got, outs[not tiled])
+
+
 def test_prefill_f32_matches_the_vector_kernel(device):
     """The matrix-core and vector fp32 paths agree to the fp32 bound on the same batch."""
     c = _case(8, 2, 128, 16, [200, 31, 64], 16, seed=3)
