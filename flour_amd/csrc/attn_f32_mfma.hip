@@ -502,14 +502,14 @@ bool prefill_f32_mfma_supported(int dtype, int head_dim, int num_seqs, int max_s
 }
 
 // The caller checks prefill_f32_mfma_supported, the 16-byte alignment of q, the pools and out
-// and of their row and head strides.
+// and of their row and head strides. kv_cap bounds the kv lengths (for the choice of the kernel).
 int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh, const void* q,
                             int64_t q_st, int64_t q_sh, const void* k_pool, const void* v_pool,
                             const int32_t* cu_seqlens_q, const int32_t* q_rows,
                             const int32_t* kv_lens, const int32_t* block_tables, int max_blocks,
-                            int num_seqs, int max_seqlen_q, int total_q, int num_heads, int n_rep,
-                            int head_dim, int block_size, int64_t num_slots, float scale,
-                            hipStream_t stream) {
+                            int num_seqs, int max_seqlen_q, int total_q, int64_t kv_cap,
+                            int num_heads, int n_rep, int head_dim, int block_size,
+                            int64_t num_slots, float scale, hipStream_t stream) {
     const int n_qt = (max_seqlen_q + F32M_QT - 1) / F32M_QT;
     if (n_qt == 0 || num_seqs == 0) return FLOUR_OK;
     const dim3 grid((unsigned)num_heads, (unsigned)num_seqs, (unsigned)n_qt);
@@ -522,7 +522,7 @@ int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh
     //    1 x 6,190 (3.0) 697 / 758. From 2.5, 4 with such a slot or with 128-row items.
     //  * Rows per sequence: 16 / 16 of 128 (128-row items), 32 x 132 rows 94 / 143, 32 x 324 325 / 354,
     //    8 x 1,296 848 / 742. At least 64, 128 and 640.
-    //  * The longest item that the block table allows, which the host cannot tell from a cached prefix
+    //  * The longest item that kv_cap (the block table's width, if no better) allows, which the host cannot tell from a cached prefix
     //    of all: up to 1.5 times a CU's share of the rows' own causal ranges. 28 / 4 of 128, 64 x 42
     //    rows, one behind 4,096 tokens 308 / 610; 32 / 8 of 128, 1 x 2,075 behind 2,048 1,096 / 1,175.
     // Of 21,095 batches with and without prefixes, some of one sequence alone, this takes 7,337: 7 of
@@ -537,7 +537,6 @@ int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh
     const int64_t full = per_row * (total_q / rows);  // items of full tiles
     const bool spare = n_rep % hw != 0;               // slots without a head
     const int mean = total_q / num_seqs;
-    const int64_t kv_cap = (int64_t)max_blocks * block_size;
     const bool wanted = 2 * full >= (spare || rows == 128 ? 8 : 5) * cus &&
                         mean >= (rows == 128 ? 640 : spare ? 128 : 64) &&
                         4 * kv_cap * cus <= 3 * full * mean;

@@ -351,6 +351,12 @@ int paged_decode_write_kv(void* out, int out_dtype, const void* q, void* k_pool,
                           float scale, int dtype, void* workspace, size_t workspace_bytes,
                           const void* k_new, const void* v_new, int64_t new_stride_tok,
                           int64_t new_stride_head, const int32_t* new_slots, void* stream);
+// Varlen prefill with what the C entry does not carry. q_rows (or null): sequence s takes its q / out
+// rows from row q_rows[s] on (its row count still cu_seqlens_q[s + 1] - cu_seqlens_q[s]): the
+// multi-row sequences of a mixed continuous-batching step, whose packed rows sit among one-row
+// sequences' rows; matrix-core shapes only (FLOUR_ERR_UNSUPPORTED otherwise, before any launch).
+// max_kv: a bound on kv_lens, which picks the kernel where the table's width would not tell a long
+// cached prefix from none; no result depends on it.
 int varlen_prefill_rows(void* out, int out_dtype, int64_t o_stride_tok, int64_t o_stride_head,
                         const void* q, int64_t q_stride_tok, int64_t q_stride_head,
                         const void* k_pool, const void* v_pool, const int32_t* cu_seqlens_q,
@@ -358,6 +364,6 @@ int varlen_prefill_rows(void* out, int out_dtype, int64_t o_stride_tok, int64_t 
                         const int32_t* block_tables, int max_blocks_per_seq, int num_seqs,
                         int max_seqlen_q, int total_q, int num_heads, int kv_heads, int head_dim,
                         int block_size, int64_t num_slots, float scale, int dtype,
-                        void* workspace, size_t workspace_bytes, void* stream);
+                        void* workspace, size_t workspace_bytes, int max_kv, void* stream);
 
 }  // namespace flour

@@ -67,9 +67,10 @@ struct KvBatchImpl {
     bool planned = false, plan_decode = false;
     int plan_n = 0, plan_total = 0, plan_max_q = 0, plan_max_ctx = 0;
     // mixed step: n_dec one-row sequences (longest context dec_max_ctx) and the longer ones
-    // (pf_max_q rows at most, pf_total in all)
+    // (pf_max_q rows at most, pf_total in all, longest context pf_max_ctx)
     bool plan_mixed = false;
     int plan_n_dec = 0, plan_dec_max_ctx = 0, plan_pf_max_q = 0, plan_pf_total = 0;
+    int plan_pf_max_ctx = 0;
     // decode step whose new positions all sit in blocks held by their sequence alone (reference
     // count 1), so no other sequence of the step reads them: the fused KV write may run
     bool plan_private = false;
@@ -350,7 +351,7 @@ struct KvBatchImpl {
         }
         // mixed step: the one-row sequences first (a decode batch), then the others (a prefill
         // batch), each entry with its first packed row
-        int n_dec = 0, dec_max_ctx = 0, pf_max_q = 0;
+        int n_dec = 0, dec_max_ctx = 0, pf_max_q = 0, pf_max_ctx = 0;
         for (int i = 0; i < n; i++) n_dec += q[i] == 1;
         const bool mixed = n_dec > 0 && n_dec < n;
         if (mixed) {
@@ -371,6 +372,7 @@ struct KvBatchImpl {
                 } else {
                     mcu[j - n_dec + 1] = mcu[j - n_dec] + q[i];
                     pf_max_q = std::max(pf_max_q, q[i]);
+                    pf_max_ctx = std::max(pf_max_ctx, lens[i]);
                 }
             }
         }
@@ -399,6 +401,7 @@ struct KvBatchImpl {
         plan_n_dec = n_dec;
         plan_dec_max_ctx = dec_max_ctx;
         plan_pf_max_q = pf_max_q;
+        plan_pf_max_ctx = pf_max_ctx;
         plan_pf_total = (int)(total - n_dec);
         plan_private = decode;
         for (int i = 0; i < n && plan_private; i++) {
@@ -675,7 +678,7 @@ extern "C" int flour_kv_batch_attention(flour_kv_batch* b, int layer, const void
             x.d_mlens() + x.plan_n_dec, x.d_mtab() + (int64_t)x.plan_n_dec * x.max_blocks,
             x.max_blocks, n_pf, x.plan_pf_max_q, x.plan_pf_total, num_heads, x.kv_heads,
             x.head_dim, x.block_size, x.num_slots, scale, x.dtype, x.d_pf_ws, x.pf_ws_bytes,
-            stream);
+            x.plan_pf_max_ctx, stream);
         if (rc == FLOUR_OK)
             return paged_decode_rows(out, out_dtype, q, x.k_pools[layer], x.v_pools[layer],
                                      x.d_mtab(), x.max_blocks, x.d_mlens(), x.d_mrows(),
@@ -685,13 +688,12 @@ extern "C" int flour_kv_batch_attention(flour_kv_batch* b, int layer, const void
         if (rc != FLOUR_ERR_UNSUPPORTED) return rc;
         clear_error();  // nothing launched: every row through the prefill kernel
     }
-    return flour_hip_varlen_prefill_ws(out, out_dtype, o_stride_tok, o_stride_head, q,
-                                       q_stride_tok, q_stride_head, x.k_pools[layer],
-                                       x.v_pools[layer], x.d_cu(), x.d_lens(), x.d_tables(),
-                                       x.max_blocks, x.plan_n, x.plan_max_q, x.plan_total,
-                                       num_heads, x.kv_heads, x.head_dim, x.block_size,
-                                       x.num_slots, scale, x.dtype, x.d_pf_ws, x.pf_ws_bytes,
-                                       stream);
+    return varlen_prefill_rows(out, out_dtype, o_stride_tok, o_stride_head, q, q_stride_tok,
+                               q_stride_head, x.k_pools[layer], x.v_pools[layer], x.d_cu(),
+                               nullptr, x.d_lens(), x.d_tables(), x.max_blocks, x.plan_n,
+                               x.plan_max_q, x.plan_total, num_heads, x.kv_heads, x.head_dim,
+                               x.block_size, x.num_slots, scale, x.dtype, x.d_pf_ws, x.pf_ws_bytes,
+                               x.plan_max_ctx, stream);
 }
 extern "C" int flour_kv_batch_write_kv_attention(flour_kv_batch* b, int layer, const void* k,
                                                  const void* v, int64_t kv_stride_tok,

@@ -734,12 +734,11 @@ extern "C" int flour_kv_cache_attention(flour_kv_cache* c, int layer, const void
                                       x.kv_heads, x.head_dim, x.block_size, x.num_slots, len,
                                       scale, x.dtype, x.d_ws, x.ws_bytes, stream);
     }
-    return flour_hip_varlen_prefill_ws(out, out_dtype, o_stride_tok, o_stride_head, q,
-                                       q_stride_tok, q_stride_head, x.k_pools[layer],
-                                       x.v_pools[layer], x.d_cu(), x.d_kv_len(), x.d_table(),
-                                       max_blocks, 1, seq_q, seq_q, num_heads, x.kv_heads,
-                                       x.head_dim, x.block_size, x.num_slots, scale, x.dtype,
-                                       x.d_pf_ws, x.pf_ws_bytes, stream);
+    return varlen_prefill_rows(out, out_dtype, o_stride_tok, o_stride_head, q, q_stride_tok,
+                               q_stride_head, x.k_pools[layer], x.v_pools[layer], x.d_cu(),
+                               nullptr, x.d_kv_len(), x.d_table(), max_blocks, 1, seq_q, seq_q,
+                               num_heads, x.kv_heads, x.head_dim, x.block_size, x.num_slots, scale,
+                               x.dtype, x.d_pf_ws, x.pf_ws_bytes, len, stream);
 }
 
 extern "C" int flour_kv_cache_reset_sequence(flour_kv_cache* c) {

@@ -313,7 +313,7 @@ static int64_t thin_items(int slots, int num_seqs, int total_q, int num_heads, i
 // CU, then four up to one, whatever the kv lengths. us there / here: 14 / 2 heads, 1 x 1,000 rows 29.6
 // / 20.7, 1 x 2,000 51.2 / 44.4; 8 / 8 heads, 1 x 2,000 50.2 / 32.5; 32 / 32, 3 x U[64, 512] 17.6 /
 // 13.3; 32 / 8, 4 x 191 behind 4,096 tokens 95 / 79; past that line 14 / 2, 16 x U[64, 286] behind
-// 1,024 35 / 47. A single prompt without a prefix (by the width of its block table) has items of every
+// 1,024 35 / 47. A single prompt without a prefix (by kv_cap) has items of every
 // length, which the snake pairs: two slots up to one item per CU at four (1 x 2,000 rows 39.9 against
 // 44.4 with four), four up to one and a half (1 x 2,867 rows 66.7 there, 58.8 here). Of
 // 21,794 batches of 1-64 sequences behind 0-4,096 tokens one is more than 3% slower than there (4%).
@@ -321,7 +321,7 @@ static int64_t thin_items(int slots, int num_seqs, int total_q, int num_heads, i
 // 20.8 / 21.2; 1 x 2,000 74 / 79; only 1 x 256 gained, 17.0 / 15.6).
 static int g_prefill_small = 1;  // a test / tuning switch
 
-// kv_cap: the positions that a row of the block table holds.
+// kv_cap: a bound on the kv lengths (the positions that a row of the block table holds, or less).
 int prefill_thin_slots(int num_seqs, int max_seqlen_q, int total_q, int64_t kv_cap, int num_heads,
                        int n_rep, int head_dim, int cus) {
     if (g_prefill_small == 0 || head_dim != PT_D || num_seqs > 64 || max_seqlen_q > 65536) return 0;

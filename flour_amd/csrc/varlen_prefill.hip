@@ -54,9 +54,9 @@ int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh
                             int64_t q_st, int64_t q_sh, const void* k_pool, const void* v_pool,
                             const int32_t* cu_seqlens_q, const int32_t* q_rows,
                             const int32_t* kv_lens, const int32_t* block_tables, int max_blocks,
-                            int num_seqs, int max_seqlen_q, int total_q, int num_heads, int n_rep,
-                            int head_dim, int block_size, int64_t num_slots, float scale,
-                            hipStream_t stream);
+                            int num_seqs, int max_seqlen_q, int total_q, int64_t kv_cap,
+                            int num_heads, int n_rep, int head_dim, int block_size,
+                            int64_t num_slots, float scale, hipStream_t stream);
 int prefill_thin_slots(int num_seqs, int max_seqlen_q, int total_q, int64_t kv_cap, int num_heads,
                        int n_rep, int head_dim, int cus);
 int launch_prefill_thin(int dtype, int out_dtype, void* out, int64_t o_st, int64_t o_sh,
@@ -1726,7 +1726,7 @@ static int varlen_prefill_impl(void* out, int out_dtype, int64_t o_stride_tok,
                                int max_seqlen_q, int total_q, int num_heads, int kv_heads,
                                int head_dim, int block_size, int64_t num_slots, float scale,
                                int dtype, void* workspace, size_t workspace_bytes,
-                               const int32_t* q_rows, void* stream) {
+                               const int32_t* q_rows, int max_kv, void* stream) {
     clear_error();
     if (!valid_dtype(dtype) || !valid_dtype(out_dtype)) {
         set_error("varlen_prefill: unknown dtype (%d, out %d)", dtype, out_dtype);
@@ -1748,6 +1748,7 @@ static int varlen_prefill_impl(void* out, int out_dtype, int64_t o_stride_tok,
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int n_rep = num_heads / kv_heads;
+    const int64_t kv_cap = std::min<int64_t>((int64_t)max_blocks_per_seq * block_size, max_kv);
     const int es = elem_bytes(dtype);
     const int oes = elem_bytes(out_dtype);
     const bool aligned = ((uintptr_t)q % 16 == 0) && ((uintptr_t)k_pool % 16 == 0) &&
@@ -1763,7 +1764,7 @@ static int varlen_prefill_impl(void* out, int out_dtype, int64_t o_stride_tok,
         return launch_prefill_f32_mfma(out_dtype, out, o_stride_tok, o_stride_head, q, q_stride_tok,
                                        q_stride_head, k_pool, v_pool, cu_seqlens_q, nullptr,
                                        kv_lens, block_tables, max_blocks_per_seq, num_seqs,
-                                       max_seqlen_q, total_q, num_heads, n_rep, head_dim,
+                                       max_seqlen_q, total_q, kv_cap, num_heads, n_rep, head_dim,
                                        block_size, num_slots, scale, s);
     if (!mfma && q_rows) {
         set_error("varlen_prefill: row indices need the matrix-core path");
@@ -1785,8 +1786,7 @@ static int varlen_prefill_impl(void* out, int out_dtype, int64_t o_stride_tok,
     // small batches at head_dim 64: more, shorter items
     const int slots = g_prefill_pv_mode == PV_F16
                           ? prefill_thin_slots(num_seqs, max_seqlen_q, total_q,
-                                               (int64_t)max_blocks_per_seq * block_size, num_heads,
-                                               n_rep, head_dim, device_cus())
+                                               kv_cap, num_heads, n_rep, head_dim, device_cus())
                           : 0;
     if (slots)
         return launch_prefill_thin(dtype, out_dtype, out, o_stride_tok, o_stride_head, q,
@@ -1836,7 +1836,7 @@ extern "C" int flour_hip_varlen_prefill(void* out, int out_dtype, int64_t o_stri
                                q_stride_head, k_pool, v_pool, cu_seqlens_q, kv_lens, block_tables,
                                max_blocks_per_seq, num_seqs, max_seqlen_q, total_q, num_heads,
                                kv_heads, head_dim, block_size, num_slots, scale, dtype, nullptr, 0,
-                               nullptr, stream);
+                               nullptr, INT_MAX, stream);
 }
 
 extern "C" int flour_hip_varlen_prefill_workspace_size(int num_seqs, int max_blocks_per_seq,
@@ -1882,15 +1882,11 @@ extern "C" int flour_hip_varlen_prefill_ws(void* out, int out_dtype, int64_t o_s
                                q_stride_head, k_pool, v_pool, cu_seqlens_q, kv_lens, block_tables,
                                max_blocks_per_seq, num_seqs, max_seqlen_q, total_q, num_heads,
                                kv_heads, head_dim, block_size, num_slots, scale, dtype, workspace,
-                               workspace_bytes, nullptr, stream);
+                               workspace_bytes, nullptr, INT_MAX, stream);
 }
 
 namespace flour {
 
-// Varlen prefill whose sequence s takes its q / out rows from row q_rows[s] on (its row count
-// still cu_seqlens_q[s + 1] - cu_seqlens_q[s]): the multi-row sequences of a mixed
-// continuous-batching step, whose packed rows sit among one-row sequences' rows. Matrix-core
-// shapes only (FLOUR_ERR_UNSUPPORTED otherwise, before any launch).
 int varlen_prefill_rows(void* out, int out_dtype, int64_t o_stride_tok, int64_t o_stride_head,
                         const void* q, int64_t q_stride_tok, int64_t q_stride_head,
                         const void* k_pool, const void* v_pool, const int32_t* cu_seqlens_q,
@@ -1898,16 +1894,12 @@ int varlen_prefill_rows(void* out, int out_dtype, int64_t o_stride_tok, int64_t 
                         const int32_t* block_tables, int max_blocks_per_seq, int num_seqs,
                         int max_seqlen_q, int total_q, int num_heads, int kv_heads, int head_dim,
                         int block_size, int64_t num_slots, float scale, int dtype,
-                        void* workspace, size_t workspace_bytes, void* stream) {
-    if (!q_rows) {
-        set_error("varlen_prefill_rows: null row indices");
-        return FLOUR_ERR_INVALID_ARGUMENT;
-    }
+                        void* workspace, size_t workspace_bytes, int max_kv, void* stream) {
     return varlen_prefill_impl(out, out_dtype, o_stride_tok, o_stride_head, q, q_stride_tok,
                                q_stride_head, k_pool, v_pool, cu_seqlens_q, kv_lens, block_tables,
                                max_blocks_per_seq, num_seqs, max_seqlen_q, total_q, num_heads,
                                kv_heads, head_dim, block_size, num_slots, scale, dtype, workspace,
-                               workspace_bytes, q_rows, stream);
+                               workspace_bytes, q_rows, max_kv, stream);
 }
 
 }  // namespace flour

@@ -338,3 +338,28 @@ def test_fused_entry_point_runs_other_steps_as_two_calls(device):
         torch.cuda.synchronize()
         assert torch.equal(kp, k1) and torch.equal(vp, v1) and torch.equal(out, ref)
         check(b, 0, sids, qn, q, out, f"write + attention in one call, rows {qn}")
+
+
+@pytest.mark.parametrize("dtype,Hq,Gk,Dh,lens", [(torch.float32, 32, 8, 128, [640] * 4),
+                                                 (torch.bfloat16, 14, 2, 64, [2016])])
+def test_prefill_kernel_goes_by_the_sequences_not_the_table(device, dtype, Hq, Gk, Dh, lens):
+    """A batch's block tables are as wide as its longest allowed sequence, which would leave room for
+    long cached prefixes: the kernel is chosen by the lengths that the plan knows, so that a prefill
+    step gives varlen_prefill's result over tables of just those lengths bit for bit."""
+    b = KvBatch(1, 1024, len(lens), 8192, sum(lens), Hq, Gk, Dh, dtype, BS)
+    sids = [b.add_sequence() for _ in lens]
+    b.step(sids, lens)
+    gd = torch.Generator(device="cuda").manual_seed(14)
+    T = sum(lens)
+    k, v = (torch.randn((T, Gk, Dh), generator=gd, device="cuda").to(dtype) for _ in range(2))
+    b.write_kv(0, k, v)
+    q = torch.randn((T, Hq, Dh), generator=gd, device="cuda").to(dtype)
+    got = b.attention(0, q, SCALE, out_dtype=torch.float32)
+    bt = torch.tensor([b.blocks(s) for s in sids], dtype=torch.int32, device=device)
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device=device)
+    kl = torch.tensor(lens, dtype=torch.int32, device=device)
+    tight = ops.varlen_prefill(q, *b.pool(0), cu, kl, bt, max(lens), SCALE, out_dtype=torch.float32)
+    wide = ops.varlen_prefill(q, *b.pool(0), cu, kl, torch.nn.functional.pad(bt, (0, 300)), max(lens),
+                              SCALE, out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    assert torch.equal(got, tight) and not torch.equal(got, wide)
