@@ -303,8 +303,8 @@ def test_decode_repeat_calls_reuse_workspace(device):
 @pytest.mark.parametrize("nwg", [1, 3, 7, 100, 513, 4096])
 def test_decode_workgroup_partitions_agree(device, nwg, w):
     """Any number of workgroups and any weighting of the ranges between even and odd workgroups
-    (hence any cut of the chunk list into pieces, including more workgroups than chunks and
-    empty ranges) meets the same fp32-accumulator bound."""
+    (hence any cut of the chunk list into pieces, including more workgroups than ranges of two
+    chunks) meets the same fp32-accumulator bound."""
     from flour_amd import _lib
     c = make_decode(6, 32, 8, 128, 16, (1, 5000), dtype=torch.bfloat16, seed=23, device=device,
                     context_lens=[4999, 1, 0, 33, 2048, 700])
@@ -320,6 +320,38 @@ def test_decode_workgroup_partitions_agree(device, nwg, w):
     max_abs, rel = errors(got, ref)
     assert max_abs <= 2e-3 and rel <= 1e-3
     assert not got[2].any()  # empty context
+
+
+@pytest.mark.parametrize("dt,B,tokens", [(torch.bfloat16, 64, 2400), (torch.bfloat16, 80, 2000),
+                                         (torch.float32, 64, 1200), (torch.float32, 80, 1000)])
+def test_decode_beyond_32_bit_ranges(device, dt, B, tokens):
+    """Chunks x ranges past the 32-bit arithmetic of the wave ranges (174,000 chunks on 768 waves;
+    here 38,000 on 4,096), in both kernels, with up to and more than 64 sequences. Sequences share
+    their pages."""
+    from flour_amd import _lib
+    H, G, D = 32, 8, 128
+    chunk = 16 if dt == torch.float32 else 32
+    ctx = [tokens - s for s in range(B)]
+    total = G * sum(-(-n // chunk) for n in ctx)
+    assert total * (32 * 4096 + 2 + 32) > 0xffffffff
+    g = torch.Generator(device=device).manual_seed(B)
+    kp, vp = (torch.randn((G, 4096, D), generator=g, device=device).to(dt) for _ in range(2))
+    q = torch.randn((B, H, D), generator=g, device=device).to(dt)
+    bt = torch.stack([torch.randperm(256, generator=torch.Generator().manual_seed(s))[:-(-tokens // 16)]
+                      for s in range(B)]).to(torch.int32).to(device)
+    cl = torch.tensor(ctx, dtype=torch.int32, device=device)
+    lib = _lib.lib()
+    assert lib.flour_hip_set_decode_workgroups(4096) == 0
+    try:
+        got = ops.paged_decode(q, kp, vp, bt, cl, D ** -0.5, tokens, out_dtype=torch.float32,
+                               workspace=ops.DecodeWorkspace(device))
+        torch.cuda.synchronize()
+    finally:
+        lib.flour_hip_set_decode_workgroups(0)
+    ref = O.paged_attention(to_np(q), to_np(kp), to_np(vp), to_np(bt),
+                            np.arange(B + 1, dtype=np.int32), to_np(cl), 16, D ** -0.5)
+    max_abs, rel = errors(to_np(got), ref)
+    assert max_abs <= (1e-5 if dt == torch.float32 else 2e-3) and rel <= 1e-3
 
 
 def test_decode_block_permutation_invariance(device):
