@@ -475,20 +475,6 @@ __global__ __launch_bounds__(F32T_WAVES * 64, 2) void prefill_f32_tile_kernel(
     }
 }
 
-static int device_cus_f32() {
-    static int cached[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (cached[dev] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            n <= 0)
-            n = 256;
-        cached[dev] = n;
-    }
-    return cached[dev];
-}
-
 // 0: the vector kernel, 1: by the rules below, 2 / 3: never / always (within its limits) the tile
 // kernel. A test / tuning switch.
 static int g_prefill_f32_mfma = 1;
@@ -531,7 +517,7 @@ int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh
     const int hw = item_heads(n_rep), kv_heads = num_heads / n_rep;
     const int rows = F32M_QT * (4 / hw);
     const int64_t per_row = (int64_t)kv_heads * ((n_rep + hw - 1) / hw);
-    const int64_t cus = device_cus_f32();
+    const int64_t cus = device_cus();
     const bool fits = !q_rows && num_seqs <= 64 && num_slots * head_dim * 4 <= 0x7fffffff &&
                       per_row * num_seqs * ((int64_t)max_seqlen_q / rows + 1) <= 0x3fffffff;
     const int64_t full = per_row * (total_q / rows);  // items of full tiles

@@ -354,20 +354,6 @@ __global__ __launch_bounds__(simt_max_waves(NQ) * 64) void attn_simt_kernel(
 
 static int nq_pow2(int nq) { return nq <= 1 ? 1 : nq <= 2 ? 2 : nq <= 4 ? 4 : 8; }
 
-static int device_cus_simt() {
-    static int cached[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (cached[dev] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            n <= 0)
-            n = 256;
-        cached[dev] = n;
-    }
-    return cached[dev];
-}
-
 template <typename T, int LPR, int NQ>
 static void launch_simt_t(dim3 grid, int waves, size_t lds, void* out, int out_dtype,
                           int64_t o_st, int64_t o_sh, const void* q, int64_t q_st, int64_t q_sh,
@@ -469,7 +455,7 @@ int launch_attn_simt(int dtype, int out_dtype, void* out, int64_t o_st, int64_t 
     // waves per workgroup: enough workgroups x waves for 8 waves per CU, no more waves than the
     // longest kv range has row loads for, and the merge buffer within 64 KiB of LDS
     const int64_t wgs = items * kv_heads * groups;
-    const int64_t want = (8LL * device_cus_simt() + wgs - 1) / wgs;
+    const int64_t want = (8LL * device_cus() + wgs - 1) / wgs;
     const int64_t kv_cap = std::min<int64_t>(max_kv, (int64_t)max_blocks * block_size);
     const int64_t loads = (kv_cap + (64 / lpr) * SIMT_UNROLL - 1) / ((64 / lpr) * SIMT_UNROLL);
     int waves = 1;

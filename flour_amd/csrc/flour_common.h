@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <exception>
 #include <new>
 #include <string>
@@ -283,6 +284,28 @@ __device__ __forceinline__ void store_run(void* out, int out_dtype, int64_t idx,
         else
             *reinterpret_cast<uint32_t*>(static_cast<f16_t*>(out) + idx) = pack2<f16_t>(v[0], v[1]);
     }
+}
+
+// The place of token t of 16 in a V^T row: bits 2 and 3 swapped, the order in which the score
+// registers of S^T = K Q^T hold a row's positions.
+__device__ __forceinline__ int sigma16(int t) {
+    return (t & ~12) | ((t & 4) << 1) | ((t & 8) >> 1);
+}
+
+// ------------------------------------------------------------------ host-side device facts
+// CUs of the current device (256 where it cannot be asked), looked up once per device.
+inline int device_cus() {
+    static std::atomic<int> cached[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    int n = cached[dev].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+            n <= 0)
+            n = 256;
+        cached[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
 }
 
 // ------------------------------------------------------------------ host-side error state

@@ -123,20 +123,6 @@ static int g_wg_override = 0;  // tuning / test hook: number of waves (0 = one r
 // batch 6,083 -> 6,231, head_dim-64 batch even).
 static int g_xcd_weight = 2;
 
-static int device_cus() {
-    static int cached[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (cached[dev] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            n <= 0)
-            n = 256;
-        cached[dev] = n;
-    }
-    return cached[dev];
-}
-
 static int decode_workgroups(int dtype) {
     const int per_cu = dtype == FLOUR_DTYPE_F32 ? DEC_WAVES_PER_CU_F32 : DEC_WAVES_PER_CU;
     const int n = g_wg_override > 0 ? g_wg_override : device_cus() * per_cu;

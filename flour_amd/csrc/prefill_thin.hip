@@ -74,7 +74,6 @@ __global__ __launch_bounds__(PT_WAVES * 64, 2) void prefill_thin_kernel(
     // are runs of a row (conflict-free)
     const int k_row = tid / CPR, k_col = (tid % CPR) * 8;
     const int v_tp = tid % RPP, v_col = (tid / RPP) * 8;
-    auto sigma16 = [](int t) { return (t & ~12) | ((t & 4) << 1) | ((t & 8) >> 1); };
 
     using Walk = ItemWalk<false>;
     Walk items;

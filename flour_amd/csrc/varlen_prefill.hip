@@ -163,10 +163,6 @@ static constexpr int PF_VPAGE_BYTES = 16 * PF_D * 2;
 __device__ __forceinline__ void gstore_b128(void* p, u32x4 v) {
     asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" :: "v"(p), "v"(v) : "memory");
 }
-__device__ __forceinline__ int sigma16(int t) {  // swap bits 2 and 3 (token order in V^T rows)
-    return (t & ~12) | ((t & 4) << 1) | ((t & 8) >> 1);
-}
-
 template <typename T, typename TO, int PV, bool BS16, bool DMA, int D>
 __global__ __launch_bounds__(PF_THREADS, 1) void varlen_prefill_mfma_kernel(
     TO* __restrict__ out, int64_t o_st, int64_t o_sh, const T* __restrict__ q, int64_t q_st,
@@ -1594,20 +1590,6 @@ static int g_prefill_dma = 1;
 static constexpr int PF_DMA_MIN_MEAN_Q = 1536;
 // Largest staging copy the DMA path takes; beyond it the launch uses register staging.
 static constexpr int64_t PF_STAGE_MAX_BYTES = int64_t(1) << 30;
-
-static int device_cus() {
-    static int cached[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (cached[dev] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            n <= 0)
-            n = 256;
-        cached[dev] = n;
-    }
-    return cached[dev];
-}
 
 // Bytes of the V staging copy the direct-to-LDS path reads for a call with num_seqs sequences
 // and block-table rows of max_blocks pages of block_size tokens (kv_heads heads, head_dim 128):
