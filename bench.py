@@ -487,9 +487,10 @@ def prefill_kernel_name(case) -> str:
 
     d = case.q.shape[2]
     if case.q.dtype in (torch.bfloat16, torch.float16) and d in (64, 128) and case.block_size % 16 == 0:
-        return "varlen_prefill_mfma_kernel"
+        return ("prefill_thin_kernel (small batches) or varlen_prefill_mfma_kernel" if d == 64
+                else "varlen_prefill_mfma_kernel")
     if case.q.dtype == torch.float32 and d in (64, 128):
-        return "prefill_f32_mfma_kernel (fp32 matrix cores)"
+        return "prefill_f32_mfma_kernel or prefill_f32_tile_kernel (fp32 matrix cores)"
     return "attn_simt_kernel"
 
 
@@ -499,8 +500,12 @@ def decode_kernel_name(case) -> str:
 
     B, H, D = case.q.shape
     G = case.k_pool.shape[0]
-    mfma = (case.q.dtype in (torch.bfloat16, torch.float16) and D in (64, 128) and
-            case.block_size % 16 == 0 and H // G <= 16 and B <= 4096)
+    mfma = (D in (64, 128) and case.block_size % 16 == 0 and H // G <= 16 and B <= 4096)
+    if mfma and case.q.dtype == torch.float32:
+        # (the shortest step that the library's rule splits)
+        if case.max_context_len * D * min(8, 1 << (H // G - 1).bit_length()) < 131072:
+            return "attn_simt_kernel (vector ALUs)"
+        return "paged_decode_mfma_kernel + paged_decode_merge_kernel, or attn_simt_kernel"
     return ("paged_decode_mfma_kernel + paged_decode_merge_kernel" if mfma
             else "attn_simt_kernel (vector ALUs)")
 

@@ -508,9 +508,10 @@ int launch_prefill_f32_mfma(int out_dtype, void* out, int64_t o_st, int64_t o_sh
     //    1 x 6,190 (3.0) 697 / 758. From 2.5, 4 with such a slot or with 128-row items.
     //  * Rows per sequence: 16 / 16 of 128 (128-row items), 32 x 132 rows 94 / 143, 32 x 324 325 / 354,
     //    8 x 1,296 848 / 742. At least 64, 128 and 640.
-    //  * The longest item that kv_cap (the block table's width, if no better) allows, which the host cannot tell from a cached prefix
-    //    of all: up to 1.5 times a CU's share of the rows' own causal ranges. 28 / 4 of 128, 64 x 42
-    //    rows, one behind 4,096 tokens 308 / 610; 32 / 8 of 128, 1 x 2,075 behind 2,048 1,096 / 1,175.
+    //  * The longest item that kv_cap (the block table's width, if no better) allows, since the host
+    //    cannot tell one long context from a cached prefix of all: up to 1.5 times a CU's share of the
+    //    rows' own causal ranges. 28 / 4 of 128, 64 x 42 rows, one behind 4,096 tokens 308 / 610; 32 /
+    //    8 of 128, 1 x 2,075 behind 2,048 1,096 / 1,175.
     // Of 21,095 batches with and without prefixes, some of one sequence alone, this takes 7,337: 7 of
     // them are more than 3% slower than on the other kernel, the geometric mean is 1.24x.
     // Its item list holds up to 64 sequences, its loads 32-bit offsets.

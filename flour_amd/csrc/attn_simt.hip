@@ -1,7 +1,8 @@
 // attn_simt.hip — paged attention on the vector ALUs for the calls the matrix-core kernels do
-// not take: short fp32 decode steps (fp32 is the reference's dtype when config.json names none,
-// engine.rs:32-38), head dims other than 128 (64 for Qwen2.5-0.5B-sized models) and page sizes that are not a
-// multiple of 16. Decode (seq_q == 1) and causal varlen prefill share the kernel.
+// not take: short fp32 decode steps and those without a workspace (fp32 is the reference's dtype when
+// config.json names none, engine.rs:32-38), head dims other than 64 and 128, page sizes of 16-bit
+// pools that are not a multiple of 16. Decode (seq_q == 1) and causal varlen prefill share the
+// kernel.
 //
 // Semantics follow paged_attention (src/backend/cpu.rs:57-112): query row i of a sequence with
 // q_len rows and kv_len cached positions sees kv position j iff j <= kv_len - q_len + i

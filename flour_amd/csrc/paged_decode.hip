@@ -169,14 +169,15 @@ struct WaveRanges {
     }
 };
 
-// Whether every numerator of WaveRanges fits 32 bits (as it does at any practical size).
+// Whether every numerator of WaveRanges fits 32 bits: up to ~174,500 chunks on 768 waves (64 x 10.9K
+// tokens over 8 kv heads of a 16-bit pool), ~131,000 on 1,024 (64 x 4.1K of an fp32 one).
 __device__ __forceinline__ bool ranges_narrow(int64_t total, int64_t n, int w) {
     return (uint64_t)total * (uint64_t)(32 * n + w + 32) <= 0xffffffffull;
 }
 
 // Ranges that a list of `total` chunks is cut into by a grid of `cap` waves: at least two chunks
 // each. Fewer, longer ranges leave fewer pieces to merge (one 2,000-token sequence of 8 kv heads,
-// 504 chunks: 10.2 us on 256 waves, 10.9 on 504), a list of more than `cap` chunks has a range of
+// 504 chunks: 10.2 us on 252 waves, 10.9 on 504), a list of more than `cap` chunks has a range of
 // two anyway, and no range is empty (the smallest share is (32 - w) / 32 >= 1/2 of the mean).
 __device__ __forceinline__ int64_t range_count(int64_t total, int64_t cap) {
     const int64_t half = total >> 1;

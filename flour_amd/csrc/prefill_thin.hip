@@ -10,12 +10,15 @@
 // chip has CUs and waits for one item's chain of kv tiles. Here an item is SLOTS = 4 or 2 (head,
 // 32-row block) slots of one kv head and sequence, each on 8 / SLOTS waves that take every 2nd or
 // 4th 32-position tile: two to eight times the items, and a chain half or a quarter as long. The
-// price is that K / V are staged for fewer rows at a time. A wave's step is bound by its vector
-// issue (exp2, packing, the split of P), and the batch by its longest chain of steps.
+// price is that K / V are staged for fewer rows at a time.
 //  * One workgroup per CU walks the items longest first (prefill_items.h). The K / V rows of step
-//    t + 1 are loaded while step t is computed, then written to the other LDS buffer (K rows of D
-//    + 8 elements; V transposed, token t at column sigma16(t), rows of 72 elements): one barrier a
-//    step; block ids two steps ahead.
+//    t + 1 are requested before step t is computed, then written to the other LDS buffer (K rows of D
+//    + 8 elements; V transposed, token t at column sigma16(t), rows of a step's positions + 8): one
+//    barrier a step; block ids two steps ahead.
+//  * As built, a step still waits for those rows: the wait for Q's own loads, which the compiler puts
+//    at their first use inside the step loop, counts the step's loads too (vmcnt(3) .. (0) before the
+//    four score products). A step is therefore bound by one memory round trip and the vector issue
+//    behind it (exp2, packing, the split of P), and the batch by its longest chain of steps.
 //  * S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_32x32x16, the score registers being the B operand
 //    of the second product after 16-bit packing (varlen_prefill.hip has the layouts). Over bf16 pools
 //    P is split into hi + lo bf16 parts, two products each, with V as stored: ~16 bits of P and no
@@ -305,6 +308,8 @@ static int64_t thin_items(int slots, int num_seqs, int total_q, int num_heads, i
     return (int64_t)(num_heads / n_rep) * ((n_rep + hw - 1) / hw) * (total_q / rows + num_seqs);
 }
 
+static int g_prefill_small = 1;  // a test / tuning switch
+
 // Slots per item of a small batch that runs here (varlen_prefill.hip's shape checks hold; `cus`: CUs
 // of the device), 0 where varlen_prefill.hip takes it. Over a long cached prefix all items are alike,
 // and a batch takes items per CU, rounded up, times ~12 ns a position with two slots and ~18 with
@@ -312,14 +317,12 @@ static int64_t thin_items(int slots, int num_seqs, int total_q, int num_heads, i
 // CU, then four up to one, whatever the kv lengths. us there / here: 14 / 2 heads, 1 x 1,000 rows 29.6
 // / 20.7, 1 x 2,000 51.2 / 44.4; 8 / 8 heads, 1 x 2,000 50.2 / 32.5; 32 / 32, 3 x U[64, 512] 17.6 /
 // 13.3; 32 / 8, 4 x 191 behind 4,096 tokens 95 / 79; past that line 14 / 2, 16 x U[64, 286] behind
-// 1,024 35 / 47. A single prompt without a prefix (by kv_cap) has items of every
-// length, which the snake pairs: two slots up to one item per CU at four (1 x 2,000 rows 39.9 against
-// 44.4 with four), four up to one and a half (1 x 2,867 rows 66.7 there, 58.8 here). Of
-// 21,794 batches of 1-64 sequences behind 0-4,096 tokens one is more than 3% slower than there (4%).
+// 1,024 35 / 47. A single prompt without a prefix (by kv_cap) has items of every length, which the
+// snake pairs: two slots up to one item per CU at four (1 x 2,000 rows 39.9 against 44.4 with four),
+// four up to one and a half (1 x 2,867 rows 66.7 there, 58.8 here). Of 21,794 batches of 1-64
+// sequences behind 0-4,096 tokens one is more than 3% slower than there (4%).
 // At head_dim 128 the same kernel was even (32 / 8 heads, 1 x 1,000 rows 39.9 / 39.3, 3 x U[64, 512]
-// 20.8 / 21.2; 1 x 2,000 74 / 79; only 1 x 256 gained, 17.0 / 15.6).
-static int g_prefill_small = 1;  // a test / tuning switch
-
+// 20.8 / 21.2; 1 x 2,000 74 / 79; only 1 x 256 gained, 17.0 / 15.6), with the step's wait as it is.
 // kv_cap: a bound on the kv lengths (the positions that a row of the block table holds, or less).
 int prefill_thin_slots(int num_seqs, int max_seqlen_q, int total_q, int64_t kv_cap, int num_heads,
                        int n_rep, int head_dim, int cus) {

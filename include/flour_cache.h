@@ -20,7 +20,9 @@
  * device and launches the decode (seq_q == 1) or prefill kernel.
  *
  * Conventions are those of flour_hip.h: FLOUR_OK or a negative FLOUR_ERR_* code, with the
- * message in flour_hip_last_error(). Functions of one cache must not be called concurrently.
+ * message in flour_hip_last_error(). Functions of one cache must not be called concurrently, and
+ * the work that they put on streams must not overlap in time either: a cache (like a batch below)
+ * has one device copy of its tables and one workspace for all its calls.
  * Block ids and slots are int32 (the pool holds fewer than 2^31 slots).
  */
 #ifndef FLOUR_CACHE_H

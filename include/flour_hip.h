@@ -26,8 +26,9 @@
  *     inputs exactly, with one exception: prefill over bf16 pools runs P.V on fp16 matrix
  *     cores with V converted to fp16 (exact for 2^-17 <= |v| <= 65504) and P rounded to fp16;
  *     a work item whose output is not finite or whose output block has a root mean square
- *     below 2^-25 / 5e-4 (~6e-5) is recomputed with bf16 V and P split into two bf16 parts.
- *     Decode splits P into two 16-bit parts. fp32 pools stay fp32 throughout: prefill at
+ *     below 2^-25 / 5e-4 (~6e-5) is recomputed with bf16 V and P split into two bf16 parts,
+ *     which small batches at head_dim 64 use throughout. Decode splits P into two 16-bit
+ *     parts. fp32 pools stay fp32 throughout: prefill at
  *     head_dim 64 / 128 and longer decode steps there (with a large enough workspace) run on
  *     the fp32 matrix cores, every other fp32 call on the vector ALUs.
  */
@@ -123,13 +124,16 @@ int flour_hip_rope_kv_write(void* q_out, const void* q, int64_t q_stride_tok,
  *                length above max_context_len attends the first max_context_len positions)
  *   Query head h attends kv head h / (num_heads / kv_heads) (repeat_kv, cpu.rs:5-13).
  *   scale multiplies q.k before the softmax (attention.rs:108 passes 1/sqrt(head_dim)).
- *   max_context_len bounds context_lens[] and sizes the split-context grid.
+ *   max_context_len bounds context_lens[] and sizes the split-context grid. Over fp32 pools it
+ *                also decides whether a step is split at all: a bound far above the lengths can
+ *                cost a few microseconds on short steps.
  *
  * Long contexts are split across workgroups; partial (max, sum, acc) rows and the batch's
  * per-sequence chunk prefix sums go to `workspace` (device memory, 256-byte aligned, no
  * initialisation needed) and a second kernel on the same stream merges them.
  * flour_hip_paged_decode_workspace_size gives the bytes required; calls that share a
- * workspace must not overlap in time.
+ * workspace must not overlap in time. fp32 calls without a workspace (or with a smaller one)
+ * run on the vector kernel, which needs none.
  * ---------------------------------------------------------------------------------------- */
 int flour_hip_paged_decode_workspace_size(int batch, int num_heads, int kv_heads, int head_dim,
                                           int max_context_len, size_t* bytes);
